@@ -25,7 +25,10 @@ LIB = os.path.join(HERE, "libsparc_hip.so")
 H5LIB = os.path.join(HERE, "libsparc_h5.so")
 FITSLIB = os.path.join(HERE, "libsparc_fits.so")
 HDF5_DIR = os.environ.get("SPARC_HDF5_DIR", "/opt/conda")
-SOURCES = ["api.hip", "stage.hip", "ops.hip", "damp.hip"]
+# (source, object, extra flags); the stage kernels' many instances are split
+# over four objects that compile side by side
+SOURCES = [("stage.hip", f"stage{q}.o", [f"-DSPARC_STAGE_PART={q}"]) for q in range(4)] + [
+    ("api.hip", "api.o", []), ("ops.hip", "ops.o", []), ("damp.hip", "damp.o", [])]
 ARCH = os.environ.get("SPARC_OFFLOAD_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -36,9 +39,10 @@ CFLAGS = [
 ]
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *CFLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(item) -> str:
+    src, name, extra = item
+    obj = os.path.join(OBJ, name)
+    cmd = [HIPCC, *CFLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")

@@ -27,9 +27,12 @@ hipError_t launch_zpass(const StageArgs<T>& A, hipStream_t s);
 template <typename T>
 hipError_t launch_zpass_batch(const StageArgs<T>* runs, const int* item_start, int nrun, int nblk,
                               int* work, hipStream_t s);
-long zpass_items(int nx, int ny, int nchunk);
-int zpass_batch_blocks(bool f32, int ncu);
-bool stage_tile_supported(int tx, int ty);
+template <typename T>
+int zpass_batch_blocks(int ncu);
+template <typename T>
+int zpass_resident(int ncu);
+template <typename T>
+int stage_resident(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma);
 template <typename T>
 hipError_t launch_filter(int axis, int g, const T* in, T* out, int nx, int ny, int nz, long fs,
                          int nfield, int periodic, T s, int bare, hipStream_t st, const int* halt,
@@ -50,7 +53,8 @@ template <typename T>
 hipError_t launch_stage_batch(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty,
                               const StageArgs<T>* runs, const int* item_start, int nrun, int nblk,
                               int* work, hipStream_t s, bool dma);
-int stage_batch_blocks(bool f32, bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma);
+template <typename T>
+int stage_batch_blocks(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma);
 hipError_t launch_diag_reduce_batch(const void* jobs, int njobs, hipStream_t st);
 hipError_t launch_tick(int* c, int reset, hipStream_t st);
 hipError_t launch_copy(const void* in, void* out, long n, bool f32, hipStream_t st, const int* halt);
@@ -150,6 +154,8 @@ struct sparc_ctx {
   double dimc = 1.0, dimrho = 1.0;
   int tx = 64, ty = 8, kc = 8, ntx = 1, nty = 1, nchunk = 1;
   int zkc = 8, znchunk = 1;  // z-pass chunking
+  bool kc_auto = true;       // kc follows auto_chunk
+  int ncu = 256;
   bool bg_set = false, state_set = false;
   // the uploaded rhoinv is bitwise 1/rho0 (initialize.f90:1012) at every point
   bool rinv_rho0 = false;
@@ -160,6 +166,14 @@ struct sparc_ctx {
   long tcount[5] = {0, 0, 0, 0, 0};
   double tms[5] = {0, 0, 0, 0, 0};
 };
+
+// The tile shapes (in lanes) the stage kernels are built for.
+static bool stage_tile_supported(int tx, int ty) {
+  return (tx == 64 && (ty == 4 || ty == 8)) || (tx == 32 && (ty == 8 || ty == 16)) || (tx == 16 && ty == 16);
+}
+
+// z-pass work items: blocks of 256 columns x z chunks
+static long zpass_items(int nx, int ny, int nchunk) { return ((long)nx * ny + 255) / 256 * nchunk; }
 
 static long round_up(long v, long m) { return (v + m - 1) / m * m; }
 
@@ -249,14 +263,10 @@ static void free_all(sparc_ctx* c) {
   if (c->st) (void)hipStreamDestroy(c->st);
 }
 
-// Tile choice.  Shapes (in lanes) the stage kernel is built for, in order of
-// preference per variant (measured on MI355X, 512x512x300 quiet and 256^3
-// MHD: quiet FP64 and FP32 run fastest at 32x8, the MHD xy kernel at 32x16
-// in FP64, at 32x8 in FP32 with one point per lane and at 16x16 with two).
-// The first shape that fits the grid (one-sided closures need >= 6 rows in
-// the last tile of a non-periodic axis) is taken.  The z chunk is sized so
-// the launch has >= ~2048 blocks (quiet) or ~8192 (MHD xy kernel) without
-// dropping below 4 planes per block.
+// Tile choice: the shapes (in lanes) the stage kernel is built for, per
+// variant in order of preference (measured on MI355X).  A shape fits a grid if
+// the last tile of a non-periodic axis holds the >= 6 rows its one-sided
+// closures need.
 static bool tile_fits(const sparc_ctx* c, int tx, int ty) {
   if (!stage_tile_supported(tx, ty)) return false;
   if (c->cfg.periodic) return true;
@@ -264,6 +274,7 @@ static bool tile_fits(const sparc_ctx* c, int tx, int ty) {
   return ty >= 6 && !(rx > 0 && rx < 6) && !(ry > 0 && ry < 6);
 }
 
+static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost);
 static void set_geometry(sparc_ctx* c, int tx, int ty, int kc);
 
 static void choose_tile(sparc_ctx* c) {
@@ -271,7 +282,7 @@ static void choose_tile(sparc_ctx* c) {
   int tx = q.tile[0], ty = q.tile[1];
   if (!(tx > 0 && ty > 0 && stage_tile_supported(tx, ty))) {
     static const int quiet64[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
-    static const int quiet32[4][2] = {{32, 8}, {64, 4}, {16, 16}, {32, 16}};
+    static const int quiet32[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
     static const int mhd64[4][2] = {{16, 16}, {32, 16}, {32, 8}, {64, 4}};
     static const int mhd32[4][2] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
     // two points per lane (FP32, even nx): the MHD xy kernel at 16x16 lanes
@@ -280,23 +291,75 @@ static void choose_tile(sparc_ctx* c) {
                                  : (c->f32 ? quiet32 : quiet64);
     tx = 32;
     ty = 8;
+    double least = 1e300;
     for (int n = 0; n < 4; ++n) {
       // narrow grids: a 16-wide tile wastes less of each block
       if (c->nx <= 16 && pref[n][0] * c->vw > 16) continue;
-      if (tile_fits(c, pref[n][0], pref[n][1])) {
+      if (!tile_fits(c, pref[n][0], pref[n][1])) continue;
+      // the MHD shapes in order of preference; a quiet run takes the shape
+      // whose launch is shortest (auto_chunk), the preferred of equal ones
+      double cost = 0.0;
+      if (!c->mhd) auto_chunk(c, pref[n][0], pref[n][1], &cost);
+      if (cost < least) {
+        least = cost;
         tx = pref[n][0];
         ty = pref[n][1];
-        break;
       }
+      if (c->mhd) break;
     }
-    // quiet: the kernel runs fastest with about 512 blocks of full-depth
-    // chunks; a plane of more than 512 tiles of 32x8 takes 32x16 tiles
-    // instead (512x512x300 FP64, one stage: 32x8 2.61 ms at 150-plane
-    // chunks, 2.53 ms at 300; 32x16 2.22 ms at 300)
+    // a plane of more than 512 tiles of 32x8 takes 32x16 tiles, which re-read
+    // fewer halo rows (512x512x300 FP64, one stage in 300-plane chunks: 32x8
+    // 2.31 ms, 32x16 2.04 ms)
     const long t32x8 = (long)((c->nx + 32 * c->vw - 1) / (32 * c->vw)) * ((c->ny + 7) / 8);
-    if (!c->mhd && tx == 32 && ty == 8 && t32x8 > 512 && tile_fits(c, 32, 16)) ty = 16;
+    if (!c->mhd && ty == 8 && t32x8 > 512 && tile_fits(c, 32, 16)) ty = 16;
   }
   set_geometry(c, tx, ty, q.tile[2]);
+}
+
+// Planes per z chunk for a launch of one block per (tile, chunk), of which
+// `places` are resident at once: a launch takes ceil(blocks / places) rounds,
+// and a block the time of its planes plus c0 planes for its start (window
+// warm-up, staging plan), so the chunk depth with the least rounds * (kc + c0)
+// is taken, the deeper of equal ones, up to kmax planes.  A last round that is
+// nearly empty costs a whole one: 384x384x160 quiet, one stage, FP64 32x16
+// tiles on 256 places 876 us at 90 planes (576 blocks: 3 rounds of 94) and
+// 731 at 32 (1440: 6 of 36); FP32 569 -> 373; 160x160x128 FP64 147 us at 25
+// planes (600 blocks on 512 places), 104 at 26 (500).
+static int balanced_chunk(long tiles, int nz, long places, double c0, int kmax, double* cost) {
+  int best = 1;
+  double least = 1e300;
+  for (int n = 1; n <= nz; ++n) {
+    const int kc = (nz + n - 1) / n;
+    if (kc > kmax) continue;
+    const long rounds = (tiles * ((nz + kc - 1) / kc) + places - 1) / places;
+    const double t = (double)rounds * (kc + c0);
+    if (t < least) {
+      least = t;
+      best = kc;
+    }
+  }
+  if (cost) *cost = least;
+  return best;
+}
+
+// Automatic z chunk of the stage kernel on tx x ty tiles; cost: see
+// balanced_chunk (comparable between tile shapes of a variant).
+//  quiet: the window re-reads 10 planes of two fields per chunk, and a start
+//    takes as long as 4 planes (fitted over 48x48x96 .. 512x512x300);
+//  quiet with x and y CPML: the tiles at the sides take longer than the inner
+//    ones, and chunks of at most 10 planes even that out (192x192x128 FP64
+//    350 us at 36 planes, 239 at 10);
+//  MHD xy kernel: no window, half a plane to start; at most 6 planes, so the
+//    halo rows are still in L2 when the neighbouring tiles read them (256^3
+//    FP64 1484 us at 4 planes, 1473 at 6, 1515 at 12; 64x128x160 FP32, where
+//    5 planes make one round of 512 blocks, 101 us at 4 and 78 at 5).
+static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost) {
+  const long tiles = (long)((c->nx + tx * c->vw - 1) / (tx * c->vw)) * ((c->ny + ty - 1) / ty);
+  const bool dma = c->dma && tx == 16 && ty == 16;
+  const int places = c->f32 ? stage_resident<float>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma)
+                            : stage_resident<double>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma);
+  if (c->zp) return balanced_chunk(tiles, c->nz, places, 0.5, c->f32 ? 5 : 6, cost);
+  return balanced_chunk(tiles, c->nz, places, 4.0, c->cfg.use_hpml ? 10 : c->nz, cost);
 }
 
 // Tile shape, z chunk (kc <= 0: automatic) and the z pass's chunking.
@@ -305,29 +368,21 @@ static void set_geometry(sparc_ctx* c, int tx, int ty, int kc) {
   c->ty = ty;
   c->ntx = (c->nx + tx * c->vw - 1) / (tx * c->vw);
   c->nty = (c->ny + ty - 1) / ty;
-  long tiles = (long)c->ntx * c->nty;
-  if (kc <= 0) {
-    // the quiet kernel re-reads 10 planes of its z queue per chunk, so it
-    // keeps chunks deep (~512 blocks: 512x512x300 FP32 32x8 lanes, one stage
-    // 1.41 ms at 2048 blocks, 1.30 at 1024, 1.23 at 512); the MHD xy kernel
-    // has no queue and runs fastest with many shallow chunks (4 planes,
-    // measured on 256^3: 16x16 FP64 1.85 ms at 8 planes, 1.77 ms at 4)
-    // small grids: 2-plane chunks (64x64x128 quiet, one step: FP64 32x8
-    // 0.192 ms at 4 planes, 0.184 at 2, 0.198 at 1; FP32 0.171 / 0.119 /
-    // 0.120), so a launch still has ~512 blocks
-    long want = c->zp ? 16384 : 512;
-    kc = (int)std::max<long>(c->zp ? 4 : 2, (c->nz * tiles + want - 1) / want);
-    kc = std::min(kc, c->nz);
-  }
+  c->kc_auto = kc <= 0;
+  if (kc <= 0) kc = auto_chunk(c, tx, ty, nullptr);
   c->kc = kc;
   c->nchunk = (c->nz + kc - 1) / kc;
-  // z pass: about 512 blocks of 256 columns, at least 32 planes deep so the
-  // 10-plane queue warm-up stays a small overhead (256^3, two chunks of 128
-  // planes: FP64 0.471 ms, FP32 0.263 ms; one chunk of 256 planes, 256
-  // blocks: 0.492 / 0.391 ms; four chunks, 1024 blocks: 0.564 / 0.284 ms)
-  const long ncb = ((long)c->nx * c->ny + 255) / 256;
-  c->zkc = (int)std::min<long>(c->nz, std::max<long>(32, (c->nz * ncb + 511) / 512));
-  c->znchunk = (c->nz + c->zkc - 1) / c->zkc;
+  // z pass: blocks of 256 columns, streaming, at full rate with half the
+  // blocks that fit (one per CU in FP64, two in FP32); the 10-plane window a
+  // chunk reads first costs as much as 14 planes (fitted from 1 to 256 planes
+  // on eight grids: 63x79x101 FP64 55 us at 34 planes, 35 at 10; 256^3 FP64
+  // 423 at 128, 390 at 256, 473 at 64; 192x192x160 FP64 215 at 46, 187 at 64)
+  if (c->zp) {
+    const long ncb = ((long)c->nx * c->ny + 255) / 256;
+    const int places = (c->f32 ? zpass_resident<float>(c->ncu) : zpass_resident<double>(c->ncu)) / 2;
+    c->zkc = balanced_chunk(ncb, c->nz, std::max(1, places), 14.0, c->nz, nullptr);
+    c->znchunk = (c->nz + c->zkc - 1) / c->zkc;
+  }
 }
 
 static int check_tile(sparc_ctx* c) {
@@ -441,6 +496,11 @@ int sparc_hip_create(const sparc_cfg* cfg, sparc_ctx** out) {
     delete c;
     return fail(SPARC_E_INVALID, "one field slab must stay below 4 GiB: split the domain in z");
   }
+  if (hipSetDevice(c->dev) != hipSuccess) {
+    delete c;
+    return fail(SPARC_E_HIP, "hipSetDevice failed");
+  }
+  (void)hipDeviceGetAttribute(&c->ncu, hipDeviceAttributeMultiprocessorCount, c->dev);
   choose_tile(c);
   int rc = check_tile(c);
   if (rc) {
@@ -452,7 +512,6 @@ int sparc_hip_create(const sparc_cfg* cfg, sparc_ctx** out) {
     delete c;
     return code;
   };
-  if (hipSetDevice(c->dev) != hipSuccess) return bail(fail(SPARC_E_HIP, "hipSetDevice failed"));
   if ((rc = scratch_setup(c->dev))) return bail(rc);
   if (hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking) != hipSuccess)
     return bail(fail(SPARC_E_HIP, "hipStreamCreate failed"));
@@ -1075,20 +1134,23 @@ int sparc_hip_kernel_time(sparc_ctx* c, int kind, long* count, double* total_ms)
   return SPARC_OK;
 }
 
+// Room for the diagnostic partials of nblk blocks.
+static int grow_partial(sparc_ctx* c, long nblk) {
+  if (nblk <= c->partial_cap) return SPARC_OK;
+  if (c->partial) (void)hipFree(c->partial);
+  c->partial = nullptr;
+  c->partial_cap = 0;
+  int rc = dalloc((void**)&c->partial, sizeof(double) * 3 * nblk);
+  if (rc) return rc;
+  c->partial_cap = nblk;
+  return SPARC_OK;
+}
+
 // Re-tile a context between steps (the partial-sum buffer grows if needed).
 static int retile(sparc_ctx* c, int tx, int ty, int kc) {
   if (!tile_fits(c, tx, ty)) return fail(SPARC_E_INVALID, "tile shape unsupported or does not fit the grid");
   set_geometry(c, tx, ty, kc);
-  const long nblk = (long)c->ntx * c->nty * c->nchunk;
-  if (nblk > c->partial_cap) {
-    if (c->partial) (void)hipFree(c->partial);
-    c->partial = nullptr;
-    c->partial_cap = 0;
-    int rc = dalloc((void**)&c->partial, sizeof(double) * 3 * nblk);
-    if (rc) return rc;
-    c->partial_cap = nblk;
-  }
-  return SPARC_OK;
+  return grow_partial(c, (long)c->ntx * c->nty * c->nchunk);
 }
 
 int sparc_hip_set_tile(sparc_ctx* c, const int tile[3]) {
@@ -1189,6 +1251,7 @@ struct BatchGroup {
   bool mhd = false, bg3d = false, zp = false, dma = false;
   int vw = 1, tx = 0, ty = 0, nblk = 0, znblk = 0;
   std::vector<int> members;
+  std::vector<int> kc;         // z chunk depth per member in this batch
   std::vector<int> zkc;        // z-pass chunk depth per member in this batch
   void* args[5] = {};         // StageArgs<T>[members] per stage (device)
   int* item_start = nullptr;   // prefix of stage work items (device)
@@ -1240,6 +1303,8 @@ static int batch_upload_args(sparc_batch* b) {
         sparc_ctx* c = b->runs[r];
         fill_common<T>(c, h[q]);
         set_stage<T>(c, h[q], s);
+        h[q].kc = g.kc[q];
+        h[q].nchunk = (c->nz + g.kc[q] - 1) / g.kc[q];
         if (g.zp) {
           h[q].zkc = g.zkc[q];
           h[q].znchunk = (c->nz + g.zkc[q] - 1) / g.zkc[q];
@@ -1359,25 +1424,39 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     g->members.push_back(r);
   }
   const size_t asz = b->f32 ? sizeof(StageArgs<float>) : sizeof(StageArgs<double>);
+  std::vector<int> nblk_of(nrun, 0);  // diagnostic partials per run
   int rc;
   for (auto& g : b->groups) {
     std::vector<int> start(g.members.size() + 1, 0);
+    g.kc.assign(g.members.size(), 0);
     for (size_t q = 0; q < g.members.size(); ++q) {
-      const sparc_ctx* c = b->runs[g.members[q]];
-      start[q + 1] = start[q] + c->ntx * c->nty * c->nchunk;
+      sparc_ctx* c = b->runs[g.members[q]];
+      const int tiles = c->ntx * c->nty;
+      // the runs' items share the persistent blocks, so a run's own rounds do
+      // not matter here: 4-plane chunks (MHD xy kernel), or about 512 blocks
+      // of at least 2 planes (quiet)
+      const int want = g.zp ? 16384 : 512;
+      g.kc[q] = !c->kc_auto ? c->kc
+                            : std::min(c->nz, (int)std::max<long>(g.zp ? 4 : 2, ((long)c->nz * tiles + want - 1) / want));
+      const int items = tiles * ((c->nz + g.kc[q] - 1) / g.kc[q]);
+      if ((rc = grow_partial(c, items))) return bail(rc);
+      nblk_of[g.members[q]] = items;
+      start[q + 1] = start[q] + items;
     }
     for (int s = 0; s < 5; ++s)
       if ((rc = dalloc(&g.args[s], asz * g.members.size()))) return bail(rc);
     if ((rc = dalloc((void**)&g.item_start, sizeof(int) * start.size()))) return bail(rc);
     if (hipMemcpy(g.item_start, start.data(), sizeof(int) * start.size(), hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(SPARC_E_HIP, "item table upload failed"));
-    g.nblk = std::min(stage_batch_blocks(b->f32, g.mhd, g.bg3d, g.zp, g.vw, g.tx, g.ty, ncu, g.dma),
-                      (start.back() + 7) / 8 * 8);
+    const int places = b->f32 ? stage_batch_blocks<float>(g.mhd, g.bg3d, g.zp, g.vw, g.tx, g.ty, ncu, g.dma)
+                              : stage_batch_blocks<double>(g.mhd, g.bg3d, g.zp, g.vw, g.tx, g.ty, ncu, g.dma);
+    g.nblk = std::min(places, (start.back() + 7) / 8 * 8);
     if (g.zp) {
       // z-pass chunks sized for the whole group rather than per run: about
       // twice the resident grid in items, each chunk >= 48 planes deep (the
       // 10-plane queue warm-up is re-read per chunk)
-      g.znblk = zpass_batch_blocks(b->f32, ncu);
+      const int zplaces = b->f32 ? zpass_batch_blocks<float>(ncu) : zpass_batch_blocks<double>(ncu);
+      g.znblk = zplaces;
       long ncols = 0;
       for (int r : g.members) ncols += zpass_items(b->runs[r]->nx, b->runs[r]->ny, 1);
       const long per_run = std::max<long>(1, (2L * g.znblk + ncols - 1) / ncols);
@@ -1392,7 +1471,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
       if ((rc = dalloc((void**)&g.zitem_start, sizeof(int) * zs.size()))) return bail(rc);
       if (hipMemcpy(g.zitem_start, zs.data(), sizeof(int) * zs.size(), hipMemcpyHostToDevice) != hipSuccess)
         return bail(fail(SPARC_E_HIP, "item table upload failed"));
-      g.znblk = std::min(zpass_batch_blocks(b->f32, ncu), (zs.back() + 7) / 8 * 8);
+      g.znblk = std::min(zplaces, (zs.back() + 7) / 8 * 8);
     }
   }
   if ((rc = dalloc((void**)&b->tstep, sizeof(int)))) return bail(rc);
@@ -1404,7 +1483,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     sparc_ctx* c = b->runs[r];
     jobs[r].partial = c->partial;
     jobs[r].out = c->diag;
-    jobs[r].nblk = c->ntx * c->nty * c->nchunk;
+    jobs[r].nblk = nblk_of[r];
     jobs[r].pad_ = 0;
     jobs[r].g = guard_args(c);
   }

@@ -1175,6 +1175,12 @@ __global__ __launch_bounds__(TX* TY, (stage_waves<T, MHD, BG3D, ZP, VW>())) void
 // Variants: MHD xy kernel (z pass), fused MHD, quiet with 3-D backgrounds,
 // quiet with z profiles; two-point lanes for FP32 quiet and MHD xy only.
 // ---------------------------------------------------------------------------
+// work items of a run's z pass: column blocks x z chunks
+static long zpass_items(int nx, int ny, int nchunk) {
+  const long nxy = (long)nx * ny;
+  return (nxy + ZP_NT - 1) / ZP_NT * nchunk;
+}
+
 template <typename T, bool MHD, bool BG3D, int TX, int TY, bool ZP, int VW>
 static hipError_t launch_one(const StageArgs<T>& A, hipStream_t s) {
   const int nblk = A.nblk_xy * A.nchunk;
@@ -1247,22 +1253,20 @@ hipError_t launch_stage_batch(bool mhd, bool bg3d, bool zp, int vw, int tx, int 
 #undef SPARC_BT
 }
 
-template hipError_t launch_stage_batch<double>(bool, bool, bool, int, int, int, const StageArgs<double>*,
-                                               const int*, int, int, int*, hipStream_t, bool);
-template hipError_t launch_stage_batch<float>(bool, bool, bool, int, int, int, const StageArgs<float>*,
-                                              const int*, int, int, int*, hipStream_t, bool);
-
-// Persistent grid for a batch launch: the blocks of this kernel instance that
-// are resident at once (the runtime's occupancy for its registers and LDS),
-// rounded up to a multiple of 8 (one share per XCD).
+// Blocks of a kernel instance that are resident at once (the runtime's
+// occupancy for its registers and LDS).  resident_grid: rounded up to a
+// multiple of 8 (one share per XCD), the persistent grid of a batch launch.
 template <typename K>
-static int resident_grid(K kernel, int threads, int ncu) {
+static int resident_blocks(K kernel, int threads, int ncu) {
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess ||
       per_cu < 1)
     per_cu = 1;
-  const int n = ncu * per_cu;
-  return (n + 7) / 8 * 8;
+  return ncu * per_cu;
+}
+template <typename K>
+static int resident_grid(K kernel, int threads, int ncu) {
+  return (resident_blocks(kernel, threads, ncu) + 7) / 8 * 8;
 }
 
 template <typename T, bool MHD, bool BG3D, bool ZP, int VW>
@@ -1293,11 +1297,10 @@ static int batch_blocks_t(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, 
   return batch_blocks_tile<T, false, false, false, 1>(tx, ty, ncu);
 }
 
-int stage_batch_blocks(bool f32, bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma) {
-  if (dma)
-    return f32 ? resident_grid(k_stage_batch_dma<float>, 256, ncu) : resident_grid(k_stage_batch_dma<double>, 256, ncu);
-  return f32 ? batch_blocks_t<float>(mhd, bg3d, zp, vw, tx, ty, ncu)
-             : batch_blocks_t<double>(mhd, bg3d, zp, vw, tx, ty, ncu);
+template <typename T>
+int stage_batch_blocks(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma) {
+  if (dma) return resident_grid(k_stage_batch_dma<T>, 256, ncu);
+  return batch_blocks_t<T>(mhd, bg3d, zp, vw, tx, ty, ncu);
 }
 
 template <typename T>
@@ -1323,21 +1326,33 @@ hipError_t launch_stage(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, co
   return launch_tile<T, false, false, false, 1>(tx, ty, A, s);
 }
 
-template hipError_t launch_stage<double>(bool, bool, bool, int, int, int, const StageArgs<double>&,
-                                         hipStream_t);
-template hipError_t launch_stage<float>(bool, bool, bool, int, int, int, const StageArgs<float>&,
-                                        hipStream_t);
-
-bool stage_tile_supported(int tx, int ty) {
-  return (tx == 64 && (ty == 4 || ty == 8)) || (tx == 32 && (ty == 8 || ty == 16)) ||
-         (tx == 16 && ty == 16);
+// Blocks of a single-run launch that are resident at once.
+template <typename T, bool MHD, bool BG3D, bool ZP, int VW>
+static int resident_tile(int tx, int ty, int ncu) {
+#define SPARC_RES(X, Y) \
+  if (tx == X && ty == Y) return resident_blocks(k_stage<T, MHD, BG3D, X, Y, ZP, VW>, X * Y, ncu);
+  SPARC_RES(64, 4)
+  SPARC_RES(64, 8)
+  SPARC_RES(32, 8)
+  SPARC_RES(32, 16)
+  SPARC_RES(16, 16)
+#undef SPARC_RES
+  return ncu;
 }
-
-// z pass: work items per run (column blocks x z chunks), single-run and
-// batched launches, and the batch grid (two 256-thread blocks per CU).
-long zpass_items(int nx, int ny, int nchunk) {
-  const long nxy = (long)nx * ny;
-  return (nxy + ZP_NT - 1) / ZP_NT * nchunk;
+template <typename T>
+int stage_resident(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu, bool dma) {
+  if (dma) return resident_blocks(k_stage_dma<T>, 256, ncu);
+  if constexpr (sizeof(T) == 4) {
+    if (vw == 2) {
+      if (mhd) return resident_tile<T, true, true, true, 2>(tx, ty, ncu);
+      if (bg3d) return resident_tile<T, false, true, false, 2>(tx, ty, ncu);
+      return resident_tile<T, false, false, false, 2>(tx, ty, ncu);
+    }
+  }
+  if (mhd && zp) return resident_tile<T, true, true, true, 1>(tx, ty, ncu);
+  if (mhd) return resident_tile<T, true, true, false, 1>(tx, ty, ncu);
+  if (bg3d) return resident_tile<T, false, true, false, 1>(tx, ty, ncu);
+  return resident_tile<T, false, false, false, 1>(tx, ty, ncu);
 }
 
 template <typename T>
@@ -1355,16 +1370,36 @@ hipError_t launch_zpass_batch(const StageArgs<T>* runs, const int* item_start, i
   return hipGetLastError();
 }
 
-int zpass_batch_blocks(bool f32, int ncu) {
-  return f32 ? resident_grid(k_zpass_batch<float>, ZP_NT, ncu)
-             : resident_grid(k_zpass_batch<double>, ZP_NT, ncu);
+template <typename T>
+int zpass_resident(int ncu) {
+  return resident_blocks(k_zpass<T>, ZP_NT, ncu);
+}
+template <typename T>
+int zpass_batch_blocks(int ncu) {
+  return resident_grid(k_zpass_batch<T>, ZP_NT, ncu);
 }
 
-template hipError_t launch_zpass<double>(const StageArgs<double>&, hipStream_t);
-template hipError_t launch_zpass<float>(const StageArgs<float>&, hipStream_t);
-template hipError_t launch_zpass_batch<double>(const StageArgs<double>*, const int*, int, int, int*,
-                                               hipStream_t);
-template hipError_t launch_zpass_batch<float>(const StageArgs<float>*, const int*, int, int, int*,
-                                              hipStream_t);
+// The kernel instances are compiled in four parts (one object each, see
+// build.py): single-run and batched launches, in FP64 and FP32.
+#define SPARC_SINGLE(T)                                                                              \
+  template hipError_t launch_stage<T>(bool, bool, bool, int, int, int, const StageArgs<T>&, hipStream_t); \
+  template int stage_resident<T>(bool, bool, bool, int, int, int, int, bool);                        \
+  template hipError_t launch_zpass<T>(const StageArgs<T>&, hipStream_t);                             \
+  template int zpass_resident<T>(int);
+#define SPARC_BATCH(T)                                                                               \
+  template hipError_t launch_stage_batch<T>(bool, bool, bool, int, int, int, const StageArgs<T>*,    \
+                                            const int*, int, int, int*, hipStream_t, bool);          \
+  template int stage_batch_blocks<T>(bool, bool, bool, int, int, int, int, bool);                    \
+  template hipError_t launch_zpass_batch<T>(const StageArgs<T>*, const int*, int, int, int*, hipStream_t); \
+  template int zpass_batch_blocks<T>(int);
+#if SPARC_STAGE_PART == 0
+SPARC_SINGLE(double)
+#elif SPARC_STAGE_PART == 1
+SPARC_SINGLE(float)
+#elif SPARC_STAGE_PART == 2
+SPARC_BATCH(double)
+#else
+SPARC_BATCH(float)
+#endif
 
 }  // namespace sparc
