@@ -20,10 +20,10 @@
 
 namespace sparc {
 template <typename T>
-hipError_t launch_stage(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, const StageArgs<T>& A,
-                        hipStream_t s);
+hipError_t launch_stage(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, bool dma, int nx,
+                        const StageArgs<T>& A, T src_amp, int nblk, hipStream_t s);
 template <typename T>
-hipError_t launch_zpass(const StageArgs<T>& A, hipStream_t s);
+hipError_t launch_zpass(const StageArgs<T>& A, long nblk, hipStream_t s);
 template <typename T>
 hipError_t launch_zpass_batch(const StageArgs<T>* runs, const int* item_start, int nrun, int nblk,
                               int* work, hipStream_t s);
@@ -781,12 +781,16 @@ static void fill_common(sparc_ctx* c, StageArgs<T>& A) {
   A.kc = c->kc;
   A.fs = c->fs;
   A.ntx = c->ntx;
-  A.nty = c->nty;
   A.nblk_xy = c->ntx * c->nty;
-  A.nchunk = c->nchunk;
   A.zkc = c->zkc;
-  A.znchunk = c->znchunk;
-  A.dma = c->dma && c->tx == 16 && c->ty == 16;
+  auto lo = [&](int f) { return c->face[f].active ? c->face[f].n : 0; };
+  auto hi = [&](int f, int n) { return c->face[f].active ? c->face[f].off : n; };
+  A.xlo = lo(XBOT);
+  A.xhi = hi(XTOP, c->nx);
+  A.ylo = lo(YBOT);
+  A.yhi = hi(YTOP, c->ny);
+  A.zlo = lo(ZBOT);
+  A.zhi = hi(ZTOP, c->nz);
   A.periodic = c->cfg.periodic ? 1 : 0;
   A.pulse_dir = c->cfg.pulse_dir;
   A.rinv_rho0 = c->rinv_rho0 ? 1 : 0;
@@ -849,11 +853,14 @@ static void fill_common(sparc_ctx* c, StageArgs<T>& A) {
   A.sdep = (const T*)c->sdep;
 }
 
+// the pool buffer stage s reads
+static int stage_input(const sparc_ctx* c, int s) { return s == 1 ? c->ra : (s % 2 == 0 ? c->rk0 : c->rk1); }
+
 // Stage s of LDDRK-5: u_1 = a; stage s reads u_s and writes
 // u_{s+1} = a + beta_{s+1} K_s into the other stage buffer; stage 5 updates a.
 template <typename T>
 static void set_stage(sparc_ctx* c, StageArgs<T>& A, int s) {
-  const int uin = s == 1 ? c->ra : (s % 2 == 0 ? c->rk0 : c->rk1);
+  const int uin = stage_input(c, s);
   const int uout = s % 2 == 1 ? c->rk0 : c->rk1;
   A.first = s == 1;
   A.last = s == 5;
@@ -875,26 +882,35 @@ static GuardArgs guard_args(const sparc_ctx* c) {
 }
 
 template <typename T>
+static hipError_t enqueue_zpass(sparc_ctx* c, const StageArgs<T>& A) {
+  return launch_zpass<T>(A, zpass_items(c->nx, c->ny, c->znchunk), c->st);
+}
+template <typename T>
+static hipError_t enqueue_stage(sparc_ctx* c, const StageArgs<T>& A, double amp) {
+  return launch_stage<T>(c->mhd, c->bg3d, c->zp, c->vw, c->tx, c->ty, c->dma && c->tx == 16 && c->ty == 16,
+                         c->nx, A, (T)amp, c->ntx * c->nty * c->nchunk, c->st);
+}
+
+template <typename T>
 static int do_step(sparc_ctx* c, double amp) {
   StageArgs<T> A;
   fill_common<T>(c, A);
-  A.src_amp = (T)amp;
   for (int s = 1; s <= 5; ++s) {
     set_stage<T>(c, A, s);
     TimeRec r;
     if (c->damp) {
       // damp_velocity of this stage's vx, vy, vz (RHS.f90:166-172)
-      const hipError_t e = damp_terms(c->damp, A.u[0], c->st);
+      const hipError_t e = damp_terms(c->damp, c->pool[stage_input(c, s)], c->st);
       if (e != hipSuccess) return fail(SPARC_E_HIP, std::string("damping transforms: ") + hipGetErrorString(e));
     }
     if (c->zp) {
       timed_begin(c, 4, &r);
-      hipError_t e = launch_zpass<T>(A, c->st);
+      hipError_t e = enqueue_zpass<T>(c, A);
       timed_end(c, &r);
       if (e != hipSuccess) return fail(SPARC_E_HIP, std::string("z pass launch: ") + hipGetErrorString(e));
     }
-    timed_begin(c, A.first ? 0 : (A.last ? 2 : 1), &r);
-    hipError_t e = launch_stage<T>(c->mhd, c->bg3d, c->zp, c->vw, c->tx, c->ty, A, c->st);
+    timed_begin(c, s == 1 ? 0 : (s == 5 ? 2 : 1), &r);
+    hipError_t e = enqueue_stage<T>(c, A, amp);
     timed_end(c, &r);
     if (e != hipSuccess) return fail(SPARC_E_HIP, std::string("stage launch: ") + hipGetErrorString(e));
   }
@@ -1174,8 +1190,8 @@ static int time_middle_stage(sparc_ctx* c, int reps, double* ms) {
   hipError_t e = hipSuccess;
   for (int q = 0; q <= reps && e == hipSuccess; ++q) {
     if (q == 1) e = hipEventRecord(e0, c->st);
-    if (e == hipSuccess && c->zp) e = launch_zpass<T>(A, c->st);
-    if (e == hipSuccess) e = launch_stage<T>(c->mhd, c->bg3d, c->zp, c->vw, c->tx, c->ty, A, c->st);
+    if (e == hipSuccess && c->zp) e = enqueue_zpass<T>(c, A);
+    if (e == hipSuccess) e = enqueue_stage<T>(c, A, 0.0);
   }
   if (e == hipSuccess) e = hipEventRecord(e1, c->st);
   if (e == hipSuccess) e = hipEventSynchronize(e1);
@@ -1304,11 +1320,7 @@ static int batch_upload_args(sparc_batch* b) {
         fill_common<T>(c, h[q]);
         set_stage<T>(c, h[q], s);
         h[q].kc = g.kc[q];
-        h[q].nchunk = (c->nz + g.kc[q] - 1) / g.kc[q];
-        if (g.zp) {
-          h[q].zkc = g.zkc[q];
-          h[q].znchunk = (c->nz + g.zkc[q] - 1) / g.zkc[q];
-        }
+        if (g.zp) h[q].zkc = g.zkc[q];
         h[q].amp_tab = c->cfg.pulse_dir ? (const T*)b->amp[r] : nullptr;
         h[q].tstep = b->tstep;
       }

@@ -140,24 +140,28 @@ template <typename T> struct Face {
 // (step.f90:58) -- safe in place because a is only read at the point.
 // State arrays are given per field (the slab base of each field).
 template <typename T> struct StageArgs {
+  // What a block reads before its first loads comes first and together (one
+  // scalar load): the grid, the split, and the CPML layers' inner bounds --
+  // x < xlo or x >= xhi lies in an x face, and so on (0 and the axis' length
+  // without the face)
   int nx, ny, nz, kc;
+  int ntx, nblk_xy, periodic, pulse_dir;
+  int xlo, xhi, ylo, yhi;
+  int zlo, zhi, first, last;
   long fs;
-  int ntx, nty, nblk_xy, nchunk;
-  int zkc, znchunk;  // MHD z pass: its own z chunk (deeper: the queue warm-up re-reads 10 planes)
-  int periodic, first, last, pulse_dir;
+  const int* halt;  // the run's guard record (GuardWord below); null: no guard
+  T beta_next, dt, sxs, sys;
+  // FP32: the remainders of the FP64 values (scl above); 0 in FP64
+  T beta_lo, dt_lo, sxs_lo, sys_lo;
   // rhoinv holds 1/rho0 at every point (checked bitwise on the host), so the
   // FP64 MHD xy kernel divides (correctly rounded, the same bits) instead of
   // reading the array
   int rinv_rho0;
-  // FP64 MHD xy kernel on 16x16 tiles with even nx: stage the planes with
-  // direct-to-LDS buffer loads (k_stage_dma)
-  int dma;
-  T beta_next, dt, sxs, sys, src_amp;
-  // FP32: the remainders of the FP64 values (scl above); 0 in FP64
-  T beta_lo, dt_lo, sxs_lo, sys_lo;
+  int zkc;  // MHD z pass: its own z chunk (deeper: the queue warm-up re-reads 10 planes)
   const T* stretch_lo;  // nz remainders of stretch(k) (FP32 only)
-  // when amp_tab is set the source amplitude is amp_tab[*tstep] (a device
-  // table and step counter, so a captured step replays unchanged)
+  // batches: the source amplitude is amp_tab[*tstep] (a device table and step
+  // counter, so a captured step replays unchanged); a single run's comes with
+  // the launch
   const T* amp_tab;
   const int* tstep;
   const T* u[8];
@@ -177,8 +181,6 @@ template <typename T> struct StageArgs {
   const T *g, *stretch, *sx, *sy, *sz;
   Face<T> face[6];
   double* partial;  // last stage: 3 doubles per block (KE sum, min rho, min p)
-  // the run's guard record (Guard below); null: no guard
-  const int* halt;
 };
 
 // The stage kernels read their arguments through a pointer into the constant
@@ -208,9 +210,11 @@ template <typename T> using CPtr = const SPARC_AS4 T*;
 enum GuardWord { G_HALT = 0, G_TRIPPED = 1, G_AT = 2, G_COUNT = 3, G_MODE = 4, G_WORDS = 8 };
 enum GuardMode { GUARD_OFF = 0, GUARD_RECORD = 1, GUARD_HALT = 2 };
 
-__device__ __forceinline__ bool halted(const int* g) {
-  return g != nullptr && __atomic_load_n(g + G_HALT, __ATOMIC_RELAXED) != 0;
+// the record's halt flag (0 without a record)
+__device__ __forceinline__ int halt_word(const int* g) {
+  return g != nullptr ? __atomic_load_n(g + G_HALT, __ATOMIC_RELAXED) : 0;
 }
+__device__ __forceinline__ bool halted(const int* g) { return halt_word(g) != 0; }
 
 // Guard arguments of one run's reduction: the KE norm is
 // sqrt(sum / npts) * dimc^2 * dimrho in cgs (driver.f90:161).
@@ -347,7 +351,8 @@ template <> struct RowSumOf<F2> { using type = RowSumF2; };
 // one-sided closure differs between the lanes of a wave, so reading the
 // constant tables takes vector memory loads, and their wait also covers
 // every load in flight (the point values of the plane); LDS reads do not.
-// FP32: hi and lo of the coefficient pairs.
+// FP32: hi and lo of the coefficient pairs.  A sum over a row multiplies and
+// adds as RowSum does, in the same order.
 template <typename T> struct RowTab {
   T c[5 * 11];
   T l[sizeof(T) == 4 ? 5 * 11 : 1];
@@ -363,36 +368,6 @@ template <typename T> struct RowTab {
     }
   }
 };
-// RowSum over an LDS copy of the tables (the same products and sums)
-template <typename T> struct RowSumT {
-  const RowTab<T>& t;
-  T p = 0, s = 0;
-  __device__ __forceinline__ explicit RowSumT(const RowTab<T>& tab) : t(tab) {}
-  __device__ __forceinline__ void add(T v, int r, int m) {
-    if constexpr (sizeof(T) == 8) {
-      p += v * t.c[r * 11 + m];
-    } else {
-      p += v * t.c[r * 11 + m];
-      s += v * t.l[r * 11 + m];
-    }
-  }
-  __device__ __forceinline__ T sum() const {
-    if constexpr (sizeof(T) == 8) return p;
-    else return p + s;
-  }
-};
-struct RowSumTF2 {
-  RowSumT<float> a, b;
-  __device__ __forceinline__ explicit RowSumTF2(const RowTab<float>& tab) : a(tab), b(tab) {}
-  __device__ __forceinline__ void add(F2 v, int r, int m) {
-    a.add(v.x, r, m);
-    b.add(v.y, r, m);
-  }
-  __device__ __forceinline__ F2 sum() const { return F2(a.sum(), b.sum()); }
-};
-template <typename V> struct RowSumTOf { using type = RowSumT<V>; };
-template <> struct RowSumTOf<F2> { using type = RowSumTF2; };
-
 // point c of a lane value
 template <typename T> __device__ __forceinline__ T lane_pt(T v, int) { return v; }
 __device__ __forceinline__ float lane_pt(F2 v, int c) { return c ? v.y : v.x; }
@@ -523,6 +498,10 @@ __device__ __forceinline__ void pml_face(FR& F, uint32_t fp, V (&v)[NF], const i
       stv<CPW>(Buf<T>(F.pst + (size_t)fam[i] * n, n), fp, base[i] + beta_next * kn);
   }
 }
+
+// One period to either side, without a division: an index that is still
+// outside [0, n) lies past every cell a point of the grid reads.
+__device__ __forceinline__ int wrap1(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 __device__ __forceinline__ int wrap(int i, int n) {
   i %= n;

@@ -17,6 +17,8 @@
 // every field it feeds once).  The staging addresses, including the periodic
 // wrap, are computed once per block.  Boundary rows use the reference's
 // one-sided closures.
+#include <type_traits>
+
 #include "sparc_dev.h"
 
 namespace sparc {
@@ -43,7 +45,7 @@ constexpr int stage_waves() {
 // register queue.  VW: x points per lane (2: FP32 on even nx, F2 values); the
 // tile is TX lanes = VW*TX points wide.
 template <typename T, bool MHD, bool BG3D, int TX, int TY, bool ZP, int VW, bool DMA = false>
-__device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
+__device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical, const T src_amp) {
   static_assert(MHD || !ZP, "the z pass serves the MHD stage only");
   static_assert(!DMA || (MHD && ZP && TX == 16 && TY == 16 && VW * sizeof(T) == 8),
                 "direct-to-LDS staging: the MHD xy kernel on 16x16 tiles of 8-byte lanes");
@@ -81,8 +83,7 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
   __shared__ RowTab<T> rtab;
 
   const int tid = threadIdx.x;
-  rtab.fill(tid, NT);
-  __syncthreads();
+  const int stop = halt_word(Ap->halt);  // looked at when the first loads are on their way
   const int tx = tid % TX, ty = tid / TX;
   const int nx = Ap->nx, ny = Ap->ny, nz = Ap->nz;
   const uint32_t fs = (uint32_t)Ap->fs;
@@ -98,6 +99,15 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
   const int i = i0 + VW * tx, j = j0 + ty;
   const bool active = (i < nx) && (j < ny);
   const uint32_t ij = active ? (uint32_t)(i + nx * j) : 0u;
+
+  // What of the grid's sides this tile meets, once per work item (uniform):
+  // the x and y CPML faces, and the rows with one-sided closures.  (Asked of
+  // the arguments per plane, each face cost its own scalar round trip.)
+  const int xlo = Ap->xlo, xhi = Ap->xhi, ylo = Ap->ylo, yhi = Ap->yhi;
+  const int kzbot = Ap->zlo, kztop = Ap->zhi;
+  const int faces = (i0 < xlo ? 1 << XBOT : 0) | (i0 + TX * VW > xhi ? 1 << XTOP : 0) |
+                    (j0 < ylo ? 1 << YBOT : 0) | (j0 + TY > yhi ? 1 << YTOP : 0);
+  const bool edge_tile = !periodic && (i0 < 5 || i0 + TX * VW > nx - 5 || j0 < 5 || j0 + TY > ny - 5);
 
   // ---- staging plan: per slot the LDS cell and the global xy offset (or
   // none: outside the domain of a non-periodic axis, or past the region).
@@ -126,11 +136,10 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
     int gi = i0 / VW - HX + col, gj = j0 - 5 + row;
     bool ok = r < NR;
     if (periodic) {
-      gi = wrap(gi, nxl);
-      gj = wrap(gj, ny);
-    } else {
-      ok = ok && gi >= 0 && gi < nxl && gj >= 0 && gj < ny;
+      gi = wrap1(gi, nxl);
+      gj = wrap1(gj, ny);
     }
+    ok = ok && gi >= 0 && gi < nxl && gj >= 0 && gj < ny;
     s_ok[s] = ok;
     s_off[s] = ok ? (uint32_t)(VW * gi + nx * gj) : 0u;
     s_lds[s] = r < NR ? row * LX + col : LY * LX;
@@ -146,12 +155,19 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
   // the tile's first lane column a multiple of 16, a pair starts at an even
   // lane column, so it lies wholly inside or outside the domain and never
   // straddles a periodic wrap.
+  // The NL x NCH loads of a plane go to the block's four waves in turn: load
+  // t = wave + 4 q is chunk t % 5 of plane t / 5, so a wave's chunks come in a
+  // cycle of five (d_off holds its offsets in that order) and its q-th load
+  // takes one of two planes, chosen by a scalar select: no branches.
   constexpr int NCH = DMA ? LP / 128 : 1;
+  static_assert(!DMA || (NCH == 5 && NT == 256), "the cycle of the wave loads");
   uint32_t d_off[NCH];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if constexpr (DMA) {
     const int lane = tid & 63;
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
+    for (int q2 = 0; q2 < NCH; ++q2) {
+      const int c = (wave + 5 - q2) % 5;  // (wave + 4 q2) mod 5
       const int r = c * 128 + 2 * lane;
       int row, col;
       if (r < TY * LX) {
@@ -167,12 +183,11 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       int gi = i0 / VW - HX + col, gj = j0 - 5 + row;
       bool ok = r < NR;
       if (periodic) {
-        gi = wrap(gi, nxl);
-        gj = wrap(gj, ny);
-      } else {
-        ok = ok && gi >= 0 && gi < nxl && gj >= 0 && gj < ny;
+        gi = wrap1(gi, nxl);
+        gj = wrap1(gj, ny);
       }
-      d_off[c] = ok ? (uint32_t)(VW * gi + nx * gj) : 0xFFFFFFFFu;
+      ok = ok && gi >= 0 && gi < nxl && gj >= 0 && gj < ny;
+      d_off[q2] = ok ? (uint32_t)(VW * gi + nx * gj) : 0xFFFFFFFFu;
     }
   }
 
@@ -248,17 +263,15 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       uint32_t bo[NCH];
 #pragma unroll
       for (int c = 0; c < NCH; ++c) bo[c] = d_off[c] == 0xFFFFFFFFu ? Buf<T>::kOut : (pk + d_off[c]) * W;
-      const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
       const T* const src[NL] = {Ap->u[VX], Ap->u[VY], Ap->u[P], Ap->box, Ap->boy,
                                 Ap->boz,   Ap->u[BY], Ap->u[BZ], Ap->u[BX], Ap->u[VZ]};
+      constexpr int NLD = NL * NCH;
 #pragma unroll
-      for (int f = 0; f < NL; ++f) {
-        const Buf<T> b(src[f], fs);
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-          if ((f * NCH + c) % (NT / 64) != wave) continue;  // uniform over the wave
-          lds_load16(b.r, &LB[0][f][c * 128], bo[c]);
-        }
+      for (int q2 = 0; q2 < (NLD + 3) / 4; ++q2) {
+        if (4 * q2 + 3 >= NLD && wave + 4 * q2 >= NLD) break;  // uniform over the wave
+        const int f0 = 4 * q2 / 5, f1 = f0 + 1 < NL ? f0 + 1 : f0;
+        const T* const p = 4 * q2 % 5 + wave >= 5 ? src[f1] : src[f0];
+        lds_load16(Buf<T>(p, fs).r, &LB[0][0][0] + (wave + 4 * q2) * 128, bo[q2 % 5]);
       }
     }
   };
@@ -294,13 +307,11 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       return TY * LX + (row < 5 ? row : row - TY) * TX + (col - HX);
     }
   };
-  // 11-point derivative along x / y from LDS (derivatives.f90:38-44,66-75,92-101).
-  // x: the centred row for every point of the lane, then the one-sided rows
-  // for points within 5 of a non-periodic edge, reading the LDS row as
-  // points (point x sits at index x - i0 + VW*HX).
+  // 11-point derivative along x / y from LDS (derivatives.f90:38-44,66-75,92-101),
+  // the centred row at every point.  x: point x of a row sits at index
+  // x - i0 + VW*HX.
   auto dx_lds = [&](int f) -> V {
     const V* row = &L[f][lidx(ty + 5, 0)];
-    V out;
     if constexpr (VW == 1) {
       T acc = 0, acl = 0;
       const int c0 = tx + HX;
@@ -311,7 +322,7 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
         if constexpr (sizeof(T) == 4) acl += Coef<T>::cl(m - 1) * d;
       }
       if constexpr (sizeof(T) == 4) acc += acl;
-      out = scl(sxs, sxl, acc);
+      return scl(sxs, sxl, acc);
     } else {
       T e[14];  // points i-6 .. i+7
 #pragma unroll
@@ -335,45 +346,12 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
         a0 += l0;
         a1 += l1;
       }
-      out = V(scl(sxs, sxl, a0), scl(sxs, sxl, a1));
+      return V(scl(sxs, sxl, a0), scl(sxs, sxl, a1));
     }
-    if (!periodic && (i < 5 || i + VW - 1 >= nx - 5)) {
-      constexpr int XO = VW * HX, RW = VW * LX;
-      const T* rp = (const T*)row;
-#pragma unroll
-      for (int c = 0; c < VW; ++c) {
-        const int p = i + c;
-        RowSumT<T> acc(rtab);
-        if (p < 5) {
-#pragma unroll
-          for (int m = 0; m < 11; ++m) acc.add(rp[min(m - i0 + XO, RW - 1)], p, m);
-          set_lane_pt(out, c, scl(sxs, sxl, acc.sum()));
-        } else if (p >= nx - 5) {
-          const int r = nx - 1 - p;
-#pragma unroll
-          for (int m = 0; m < 11; ++m) acc.add(rp[min(max(nx - 1 - m - i0 + XO, 0), RW - 1)], r, m);
-          set_lane_pt(out, c, -scl(sxs, sxl, acc.sum()));
-        }
-      }
-    }
-    return out;
   };
   auto dy_lds = [&](int f) -> V {
     const V* pl = L[f];
     const int cx = tx + HX;
-    if (!periodic && j < 5) {
-      typename RowSumTOf<V>::type e(rtab);
-#pragma unroll
-      for (int m = 0; m < 11; ++m) e.add(pl[lidx(min(max(m - j0 + 5, 0), LY - 1), cx)], j, m);
-      return scl(sys, syl, e.sum());
-    }
-    if (!periodic && j >= ny - 5) {
-      const int r = ny - 1 - j;
-      typename RowSumTOf<V>::type e(rtab);
-#pragma unroll
-      for (int m = 0; m < 11; ++m) e.add(pl[lidx(min(max(ny - 1 - m - j0 + 5, 0), LY - 1), cx)], r, m);
-      return -scl(sys, syl, e.sum());
-    }
     V acc = 0;
     const int r0 = ty + 5;
     V acl = 0;
@@ -385,6 +363,74 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
     }
     if constexpr (sizeof(T) == 4) acc += acl;
     return scl(sys, syl, acc);
+  };
+  // The one-sided rows next to a non-periodic side, in tiles that meet one:
+  // the points within 5 of it replace their centred values.  A point's row of
+  // coefficients and its eleven cells are the same for every field of a
+  // direction, so they are read once and the fields follow without a branch
+  // (a branch per field and side, each with its own table reads, took 12000
+  // to 14000 cycles of a plane in the corner tiles of 128x96x96 MHD FP64,
+  // where the centred rows take 2500).  A tile that holds any of the 5 holds
+  // them all and the rows they read (tile_fits in the host code).
+  auto onesided_x = [&](const int* fld, V** out, auto nf) {
+    constexpr int NF = decltype(nf)::value;
+#pragma unroll
+    for (int c = 0; c < VW; ++c) {
+      const int p = i + c;
+      if (!(p < 5 || p >= nx - 5) || p >= nx) continue;
+      const bool low = p < 5;
+      const int r = low ? p : nx - 1 - p;
+      const int first_cell = (low ? 0 : nx - 1) - i0 + VW * HX, dir = low ? 1 : -1;
+      T ch[11], cl[sizeof(T) == 4 ? 11 : 1];
+#pragma unroll
+      for (int m = 0; m < 11; ++m) {
+        ch[m] = rtab.c[r * 11 + m];
+        if constexpr (sizeof(T) == 4) cl[m] = rtab.l[r * 11 + m];
+      }
+      const int row = lidx(ty + 5, 0) * VW;
+#pragma unroll
+      for (int q2 = 0; q2 < NF; ++q2) {
+        const T* rp = (const T*)L[fld[q2]];
+        T ph = 0, pl = 0;
+#pragma unroll
+        for (int m = 0; m < 11; ++m) {
+          const T v = rp[row + first_cell + dir * m];
+          ph += v * ch[m];
+          if constexpr (sizeof(T) == 4) pl += v * cl[m];
+        }
+        if constexpr (sizeof(T) == 4) ph += pl;
+        const T d = scl(sxs, sxl, ph);
+        set_lane_pt(*out[q2], c, low ? d : -d);
+      }
+    }
+  };
+  auto onesided_y = [&](const int* fld, V** out, auto nf) {
+    constexpr int NF = decltype(nf)::value;
+    if (!(j < 5 || j >= ny - 5)) return;
+    const bool low = j < 5;
+    const int r = low ? j : ny - 1 - j;
+    T ch[11], cl[sizeof(T) == 4 ? 11 : 1];
+    int at[11];
+#pragma unroll
+    for (int m = 0; m < 11; ++m) {
+      ch[m] = rtab.c[r * 11 + m];
+      if constexpr (sizeof(T) == 4) cl[m] = rtab.l[r * 11 + m];
+      at[m] = lidx((low ? m : ny - 1 - m) - j0 + 5, tx + HX);
+    }
+#pragma unroll
+    for (int q2 = 0; q2 < NF; ++q2) {
+      const V* pl2 = L[fld[q2]];
+      V ph = 0, pl = 0;
+#pragma unroll
+      for (int m = 0; m < 11; ++m) {
+        const V v = pl2[at[m]];
+        ph += v * V(ch[m]);
+        if constexpr (sizeof(T) == 4) pl += v * V(cl[m]);
+      }
+      if constexpr (sizeof(T) == 4) ph += pl;
+      const V d = scl(sys, syl, ph);
+      *out[q2] = low ? d : -d;
+    }
   };
 
   // z register queue: slot m holds plane k-5+m of each z-differentiated
@@ -511,20 +557,30 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
   // wait would also wait for the next plane's prefetched loads, which
   // complete in order before them.)
   const int pdir = Ap->pulse_dir;
-  V srcxy = 0;
+  V srcx = 0;
+  T srcy = 1;
   if (Ap->fmap) {
-    srcxy = ldv<V>(Buf<T>(Ap->fmap, nxy), (uint32_t)(i + nx * j) * W);
+    srcx = ldv<V>(Buf<T>(Ap->fmap, nxy), (uint32_t)(i + nx * j) * W);
   } else if (pdir >= 1 && pdir <= 3) {
-    const T amp = Ap->amp_tab ? Ap->amp_tab[*Ap->tstep] : Ap->src_amp;
-    srcxy = amp * ldv<V>(Buf<T>(Ap->sx, nx), (uint32_t)i * W) * Buf<T>(Ap->sy, ny)[j];
+    srcx = ldv<V>(Buf<T>(Ap->sx, nx), (uint32_t)i * W);
+    srcy = Buf<T>(Ap->sy, ny)[j];
   }
-
   if constexpr (SPF) pre_load(k0);
   if constexpr (PPF) point_load(k0, pn);
+  rtab.fill(tid, NT);
+  if (stop) return;  // the run's failure guard stopped it (uniform over the block)
+  __syncthreads();
   // the first plane's loads complete before the loop, so that on entry, as
   // on every later pass, the loop-top wait has only stores left to wait on
   // (vmcnt 0, expcnt and lgkmcnt not waited on)
   if constexpr (SPF) __builtin_amdgcn_s_waitcnt(0x0F70);
+  // the factors' product only now: at their loads it would have waited for
+  // every load before them
+  V srcxy = srcx;
+  if (!Ap->fmap && pdir >= 1 && pdir <= 3) {
+    const T amp = Ap->amp_tab ? Ap->amp_tab[*Ap->tstep] : src_amp;
+    srcxy = amp * srcx * srcy;
+  }
   for (int k = k0; k < k1; ++k) {
     SPARC_REFRESH(Ap);
     L = LB[NB == 2 ? (k & 1) : 0];
@@ -604,10 +660,15 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
           const int r = nz - 1 - k;
 #pragma unroll
           for (int f = 0; f < NQ; ++f) {
-            typename RowSumTOf<V>::type acc(rtab);
+            V ph = 0, pl = 0;
 #pragma unroll
-            for (int m = 0; m < 11; ++m) acc.add(q[f][m], r, (r + 16 - m) % 11);
-            dz[f] = -scl(st, stl, acc.sum());
+            for (int m = 0; m < 11; ++m) {
+              const int c = r * 11 + (r + 16 - m) % 11;
+              ph += q[f][m] * V(rtab.c[c]);
+              if constexpr (sizeof(T) == 4) pl += q[f][m] * V(rtab.l[c]);
+            }
+            if constexpr (sizeof(T) == 4) ph += pl;
+            dz[f] = -scl(st, stl, ph);
           }
         }
       }
@@ -628,6 +689,46 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
     if (active) {
       // xy derivatives and centre values from LDS
       V dvxdx = dx_lds(0), dvydy = dy_lds(1), gpx = dx_lds(2), gpy = dy_lds(2);
+      V dxf3 = 0, dyf3 = 0, dxf2 = 0, dyf1 = 0, dxby = 0, dxbz = 0, dybz = 0, dybx = 0;
+      if constexpr (MHD) {
+        // fences keep the LDS reads in flight to what the registers left
+        // hold: four derivatives', or one's of two-point lanes
+        auto fence = [&](bool group) {
+          if (group || VW == 2) __builtin_amdgcn_sched_barrier(0);
+        };
+        fence(true);
+        dxf3 = dx_lds(3);
+        fence(false);
+        dyf3 = dy_lds(3);
+        fence(false);
+        dxf2 = dx_lds(4);
+        fence(false);
+        dyf1 = dy_lds(5);
+        fence(true);
+        dxby = dx_lds(6);
+        fence(false);
+        dxbz = dx_lds(7);
+        fence(false);
+        dybz = dy_lds(7);
+        fence(false);
+        dybx = dy_lds(8);
+        fence(false);
+      }
+      if (edge_tile) {
+        if constexpr (MHD) {
+          constexpr int fx[6] = {0, 2, 3, 4, 6, 7}, fy[6] = {1, 2, 3, 5, 7, 8};
+          V* ox[6] = {&dvxdx, &gpx, &dxf3, &dxf2, &dxby, &dxbz};
+          V* oy[6] = {&dvydy, &gpy, &dyf3, &dyf1, &dybz, &dybx};
+          onesided_x(fx, ox, std::integral_constant<int, 6>{});
+          onesided_y(fy, oy, std::integral_constant<int, 6>{});
+        } else {
+          constexpr int fx[2] = {0, 2}, fy[2] = {1, 2};
+          V* ox[2] = {&dvxdx, &gpx};
+          V* oy[2] = {&dvydy, &gpy};
+          onesided_x(fx, ox, std::integral_constant<int, 2>{});
+          onesided_y(fy, oy, std::integral_constant<int, 2>{});
+        }
+      }
       const int cc = lidx(ty + 5, tx + HX);
       const V vx = L[0][cc], vy = L[1][cc];
       const V rho = PPF ? pc[0] : (MPX ? pm[0] : UF(RHO, g));
@@ -635,17 +736,9 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       // z pass output, in CPML family order: vz, p, bx, by, F2, F1
       auto DZ = [&](int f) -> V { return MPX ? pm[2 + f] : ldv<V>(Buf<T>(Ap->dz[f], fs), g * W); };
       V dvzdz = ZP ? DZ(0) : dz[0], gpz = ZP ? DZ(1) : dz[1];
-      V dxf3 = 0, dyf3 = 0, dxf2 = 0, dyf1 = 0, dxby = 0, dxbz = 0, dybz = 0, dybx = 0, bz = 0;
+      V bz = 0;
       V dzbx = 0, dzby = 0, dzf1 = 0, dzf2 = 0;
       if constexpr (MHD) {
-        dxf3 = dx_lds(3);
-        dyf3 = dy_lds(3);
-        dxf2 = dx_lds(4);
-        dyf1 = dy_lds(5);
-        dxby = dx_lds(6);
-        dxbz = dx_lds(7);
-        dybz = dy_lds(7);
-        dybx = dy_lds(8);
         bz = L[7][cc];
         if constexpr (ZP) {
           dzbx = DZ(2);
@@ -664,9 +757,9 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
 #pragma unroll
       for (int fz = ZBOT; fz <= ZTOP; ++fz) {
         if constexpr (ZP) break;
+        if (fz == ZBOT ? k >= kzbot : k < kztop) continue;
         const auto& F = Ap->face[fz];
         const int kp = k - F.off;
-        if (!F.active || kp < 0 || kp >= F.n) continue;
         const uint32_t fp = ij + nxy * (uint32_t)kp;
         if constexpr (MHD) {
           V v[6] = {gpz, dvzdz, dzf2, dzf1, dzbx, dzby};
@@ -687,8 +780,8 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       // points need not start on a lane boundary)
 #pragma unroll
       for (int fx = XBOT; fx <= XTOP; ++fx) {
+        if (!(faces & (1 << fx))) continue;
         const auto& F = Ap->face[fx];
-        if (!F.active) continue;
         if constexpr (VW == 2) {
           if (((F.n | F.off) & 1) == 0) {
             const int ip = i - F.off;
@@ -736,9 +829,10 @@ __device__ __forceinline__ void stage_item(CArgs<T> Ap, const int logical) {
       }
 #pragma unroll
       for (int fy = YBOT; fy <= YTOP; ++fy) {
+        if (!(faces & (1 << fy))) continue;
         const auto& F = Ap->face[fy];
         const int jp = j - F.off;
-        if (!F.active || jp < 0 || jp >= F.n) continue;
+        if (jp < 0 || jp >= F.n) continue;
         const uint32_t fp = (uint32_t)(i + nx * (jp + F.n * k));
         if constexpr (MHD) {
           V v[6] = {gpy, dvydy, dyf3, dyf1, dybx, dybz};
@@ -940,6 +1034,7 @@ constexpr int ZP_NT = 256;
 template <typename T>
 __device__ __forceinline__ void zpass_item(CArgs<T> Ap, const int logical) {
   constexpr int NT = ZP_NT;
+  const int stop = halt_word(Ap->halt);  // looked at when the first loads are on their way
   const int nz = Ap->nz;
   const uint32_t fs = (uint32_t)Ap->fs;
   const uint32_t nxy = (uint32_t)Ap->nx * (uint32_t)Ap->ny;
@@ -949,6 +1044,7 @@ __device__ __forceinline__ void zpass_item(CArgs<T> Ap, const int logical) {
   const bool active = col < nxy;
   const uint32_t ij = active ? col : 0u;
   const int k0 = chunk * kc, k1 = min(k0 + kc, nz);
+  const int kzbot = Ap->zlo, kztop = Ap->zhi;
   const bool first = Ap->first, last = Ap->last;
   const T dt = Ap->dt, bnext = Ap->beta_next;
   constexpr uint32_t W = sizeof(T);
@@ -982,6 +1078,7 @@ __device__ __forceinline__ void zpass_item(CArgs<T> Ap, const int logical) {
     for (int f = 0; f < 6; ++f) q[f][m] = t[f];
   }
   fetch(k0 + 5, nq);
+  if (stop) return;  // the run's failure guard stopped it (uniform over the block)
 
   for (int k = k0; k < k1; ++k) {
     SPARC_REFRESH(Ap);
@@ -1022,10 +1119,9 @@ __device__ __forceinline__ void zpass_item(CArgs<T> Ap, const int logical) {
       const uint32_t g = ij + (uint32_t)k * nxy;
 #pragma unroll
       for (int fz = ZBOT; fz <= ZTOP; ++fz) {
+        if (fz == ZBOT ? k >= kzbot : k < kztop) continue;
         const auto& F = Ap->face[fz];
-        const int kp = k - F.off;
-        if (!F.active || kp < 0 || kp >= F.n) continue;
-        const uint32_t fp = ij + nxy * (uint32_t)kp;
+        const uint32_t fp = ij + nxy * (uint32_t)(k - F.off);
         constexpr int fam[6] = {0, 1, 2, 3, 4, 5};
         pml_face<kStream>(F, fp, d, fam, first, last, bnext, dt);  // z-face CPML: used once
       }
@@ -1045,7 +1141,6 @@ __global__ __launch_bounds__(ZP_NT, 2) void k_zpass(const StageArgs<T> A) {
   const int xcd = b & 7, loc = b >> 3, base = nblk >> 3, rem = nblk & 7;
   const int logical = xcd * base + (xcd < rem ? xcd : rem) + loc;
   const CArgs<T> Ap = (CArgs<T>)__builtin_amdgcn_kernarg_segment_ptr();
-  if (halted(Ap->halt)) return;  // the run's failure guard stopped it
   zpass_item<T>(Ap, logical);
 }
 
@@ -1088,7 +1183,7 @@ __global__ __launch_bounds__(ZP_NT, 2) void k_zpass_batch(const StageArgs<T>* __
   for (int item = next_item(work, lo, hi, &slot); item >= 0; item = next_item(work, lo, hi, &slot)) {
     while (r + 1 < nrun && item_start[r + 1] <= item) ++r;
     const CArgs<T> Ap = (CArgs<T>)(runs + r);
-    if (!halted(Ap->halt)) zpass_item<T>(Ap, item - item_start[r]);
+    zpass_item<T>(Ap, item - item_start[r]);
   }
   leave(work);
 }
@@ -1097,14 +1192,12 @@ __global__ __launch_bounds__(ZP_NT, 2) void k_zpass_batch(const StageArgs<T>* __
 // ids to the 8 XCDs in turn; remap so each XCD gets a contiguous run of tiles
 // and the halos the tiles share stay in that XCD's L2.
 template <typename T, bool MHD, bool BG3D, int TX, int TY, bool ZP, int VW>
-__global__ __launch_bounds__(TX* TY, (stage_waves<T, MHD, BG3D, ZP, VW>())) void k_stage(const StageArgs<T> A) {
+__global__ __launch_bounds__(TX* TY, (stage_waves<T, MHD, BG3D, ZP, VW>())) void k_stage(
+    const StageArgs<T> A, const T src_amp) {
   const int nblk = gridDim.x, b = blockIdx.x;
   const int xcd = b & 7, loc = b >> 3, base = nblk >> 3, rem = nblk & 7;
   const int logical = xcd * base + (xcd < rem ? xcd : rem) + loc;
-  // A sits at offset 0 of the kernel-argument segment
-  const CArgs<T> Ap = (CArgs<T>)__builtin_amdgcn_kernarg_segment_ptr();
-  if (halted(Ap->halt)) return;  // the run's failure guard stopped it
-  stage_item<T, MHD, BG3D, TX, TY, ZP, VW>(Ap, logical);
+  stage_item<T, MHD, BG3D, TX, TY, ZP, VW>((CArgs<T>)__builtin_amdgcn_kernarg_segment_ptr(), logical, src_amp);
 }
 
 // The MHD xy kernel with direct-to-LDS staging (16x16 tiles of 8-byte
@@ -1119,13 +1212,11 @@ constexpr int dma_vw() {
   return sizeof(T) == 4 ? 2 : 1;
 }
 template <typename T>
-__global__ __launch_bounds__(256, 2) void k_stage_dma(const StageArgs<T> A) {
+__global__ __launch_bounds__(256, 2) void k_stage_dma(const StageArgs<T> A, const T src_amp) {
   const int nblk = gridDim.x, b = blockIdx.x;
   const int xcd = b & 7, loc = b >> 3, base = nblk >> 3, rem = nblk & 7;
   const int logical = xcd * base + (xcd < rem ? xcd : rem) + loc;
-  const CArgs<T> Ap = (CArgs<T>)__builtin_amdgcn_kernarg_segment_ptr();
-  if (halted(Ap->halt)) return;
-  stage_item<T, true, true, 16, 16, true, dma_vw<T>(), true>(Ap, logical);
+  stage_item<T, true, true, 16, 16, true, dma_vw<T>(), true>((CArgs<T>)__builtin_amdgcn_kernarg_segment_ptr(), logical, src_amp);
 }
 
 // The same, persistent over the work items of a batch group.
@@ -1141,7 +1232,7 @@ __global__ __launch_bounds__(256, 2) void k_stage_batch_dma(const StageArgs<T>* 
   for (int item = next_item(work, lo, hi, &slot); item >= 0; item = next_item(work, lo, hi, &slot)) {
     while (r + 1 < nrun && item_start[r + 1] <= item) ++r;
     const CArgs<T> Ap = (CArgs<T>)(runs + r);
-    if (!halted(Ap->halt)) stage_item<T, true, true, 16, 16, true, dma_vw<T>(), true>(Ap, item - item_start[r]);
+    stage_item<T, true, true, 16, 16, true, dma_vw<T>(), true>(Ap, item - item_start[r], T(0));
   }
   leave(work);
 }
@@ -1165,7 +1256,7 @@ __global__ __launch_bounds__(TX* TY, (stage_waves<T, MHD, BG3D, ZP, VW>())) void
     // no kernel writes the argument array while the batch runs; an item of
     // a run its failure guard stopped is skipped (uniform over the block)
     const CArgs<T> Ap = (CArgs<T>)(runs + r);
-    if (!halted(Ap->halt)) stage_item<T, MHD, BG3D, TX, TY, ZP, VW>(Ap, item - item_start[r]);
+    stage_item<T, MHD, BG3D, TX, TY, ZP, VW>(Ap, item - item_start[r], T(0));
   }
   leave(work);
 }
@@ -1175,26 +1266,19 @@ __global__ __launch_bounds__(TX* TY, (stage_waves<T, MHD, BG3D, ZP, VW>())) void
 // Variants: MHD xy kernel (z pass), fused MHD, quiet with 3-D backgrounds,
 // quiet with z profiles; two-point lanes for FP32 quiet and MHD xy only.
 // ---------------------------------------------------------------------------
-// work items of a run's z pass: column blocks x z chunks
-static long zpass_items(int nx, int ny, int nchunk) {
-  const long nxy = (long)nx * ny;
-  return (nxy + ZP_NT - 1) / ZP_NT * nchunk;
-}
-
 template <typename T, bool MHD, bool BG3D, int TX, int TY, bool ZP, int VW>
-static hipError_t launch_one(const StageArgs<T>& A, hipStream_t s) {
-  const int nblk = A.nblk_xy * A.nchunk;
-  hipLaunchKernelGGL((k_stage<T, MHD, BG3D, TX, TY, ZP, VW>), dim3(nblk), dim3(TX * TY), 0, s, A);
+static hipError_t launch_one(const StageArgs<T>& A, T src_amp, int nblk, hipStream_t s) {
+  hipLaunchKernelGGL((k_stage<T, MHD, BG3D, TX, TY, ZP, VW>), dim3(nblk), dim3(TX * TY), 0, s, A, src_amp);
   return hipGetLastError();
 }
 
 template <typename T, bool MHD, bool BG3D, bool ZP, int VW>
-static hipError_t launch_tile(int tx, int ty, const StageArgs<T>& A, hipStream_t s) {
-  if (tx == 64 && ty == 4) return launch_one<T, MHD, BG3D, 64, 4, ZP, VW>(A, s);
-  if (tx == 64 && ty == 8) return launch_one<T, MHD, BG3D, 64, 8, ZP, VW>(A, s);
-  if (tx == 32 && ty == 8) return launch_one<T, MHD, BG3D, 32, 8, ZP, VW>(A, s);
-  if (tx == 32 && ty == 16) return launch_one<T, MHD, BG3D, 32, 16, ZP, VW>(A, s);
-  if (tx == 16 && ty == 16) return launch_one<T, MHD, BG3D, 16, 16, ZP, VW>(A, s);
+static hipError_t launch_tile(int tx, int ty, const StageArgs<T>& A, T src_amp, int nblk, hipStream_t s) {
+  if (tx == 64 && ty == 4) return launch_one<T, MHD, BG3D, 64, 4, ZP, VW>(A, src_amp, nblk, s);
+  if (tx == 64 && ty == 8) return launch_one<T, MHD, BG3D, 64, 8, ZP, VW>(A, src_amp, nblk, s);
+  if (tx == 32 && ty == 8) return launch_one<T, MHD, BG3D, 32, 8, ZP, VW>(A, src_amp, nblk, s);
+  if (tx == 32 && ty == 16) return launch_one<T, MHD, BG3D, 32, 16, ZP, VW>(A, src_amp, nblk, s);
+  if (tx == 16 && ty == 16) return launch_one<T, MHD, BG3D, 16, 16, ZP, VW>(A, src_amp, nblk, s);
   return hipErrorInvalidValue;
 }
 
@@ -1304,26 +1388,26 @@ int stage_batch_blocks(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int
 }
 
 template <typename T>
-hipError_t launch_stage(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, const StageArgs<T>& A,
-                        hipStream_t s) {
+hipError_t launch_stage(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, bool dma, int nx,
+                        const StageArgs<T>& A, T src_amp, int nblk, hipStream_t s) {
   if (!lanes_ok<T>(mhd, zp, vw)) return hipErrorInvalidValue;
-  if (A.dma) {
-    if (!(mhd && zp && vw == dma_vw<T>() && tx == 16 && ty == 16 && A.nx % (2 * vw) == 0))
+  if (dma) {
+    if (!(mhd && zp && vw == dma_vw<T>() && tx == 16 && ty == 16 && nx % (2 * vw) == 0))
       return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_stage_dma<T>), dim3(A.nblk_xy * A.nchunk), dim3(256), 0, s, A);
+    hipLaunchKernelGGL((k_stage_dma<T>), dim3(nblk), dim3(256), 0, s, A, src_amp);
     return hipGetLastError();
   }
   if constexpr (sizeof(T) == 4) {
     if (vw == 2) {
-      if (mhd) return launch_tile<T, true, true, true, 2>(tx, ty, A, s);
-      if (bg3d) return launch_tile<T, false, true, false, 2>(tx, ty, A, s);
-      return launch_tile<T, false, false, false, 2>(tx, ty, A, s);
+      if (mhd) return launch_tile<T, true, true, true, 2>(tx, ty, A, src_amp, nblk, s);
+      if (bg3d) return launch_tile<T, false, true, false, 2>(tx, ty, A, src_amp, nblk, s);
+      return launch_tile<T, false, false, false, 2>(tx, ty, A, src_amp, nblk, s);
     }
   }
-  if (mhd && zp) return launch_tile<T, true, true, true, 1>(tx, ty, A, s);
-  if (mhd) return launch_tile<T, true, true, false, 1>(tx, ty, A, s);
-  if (bg3d) return launch_tile<T, false, true, false, 1>(tx, ty, A, s);
-  return launch_tile<T, false, false, false, 1>(tx, ty, A, s);
+  if (mhd && zp) return launch_tile<T, true, true, true, 1>(tx, ty, A, src_amp, nblk, s);
+  if (mhd) return launch_tile<T, true, true, false, 1>(tx, ty, A, src_amp, nblk, s);
+  if (bg3d) return launch_tile<T, false, true, false, 1>(tx, ty, A, src_amp, nblk, s);
+  return launch_tile<T, false, false, false, 1>(tx, ty, A, src_amp, nblk, s);
 }
 
 // Blocks of a single-run launch that are resident at once.
@@ -1356,8 +1440,7 @@ int stage_resident(bool mhd, bool bg3d, bool zp, int vw, int tx, int ty, int ncu
 }
 
 template <typename T>
-hipError_t launch_zpass(const StageArgs<T>& A, hipStream_t s) {
-  const long nblk = zpass_items(A.nx, A.ny, A.znchunk);
+hipError_t launch_zpass(const StageArgs<T>& A, long nblk, hipStream_t s) {
   hipLaunchKernelGGL((k_zpass<T>), dim3((unsigned)nblk), dim3(ZP_NT), 0, s, A);
   return hipGetLastError();
 }
@@ -1382,9 +1465,10 @@ int zpass_batch_blocks(int ncu) {
 // The kernel instances are compiled in four parts (one object each, see
 // build.py): single-run and batched launches, in FP64 and FP32.
 #define SPARC_SINGLE(T)                                                                              \
-  template hipError_t launch_stage<T>(bool, bool, bool, int, int, int, const StageArgs<T>&, hipStream_t); \
+  template hipError_t launch_stage<T>(bool, bool, bool, int, int, int, bool, int, const StageArgs<T>&, T, \
+                                      int, hipStream_t);                                             \
   template int stage_resident<T>(bool, bool, bool, int, int, int, int, bool);                        \
-  template hipError_t launch_zpass<T>(const StageArgs<T>&, hipStream_t);                             \
+  template hipError_t launch_zpass<T>(const StageArgs<T>&, long, hipStream_t);                             \
   template int zpass_resident<T>(int);
 #define SPARC_BATCH(T)                                                                               \
   template hipError_t launch_stage_batch<T>(bool, bool, bool, int, int, int, const StageArgs<T>*,    \
