@@ -20,8 +20,9 @@ struct DampPlan {
   hipfftHandle fwd = 0, inv = 0;
   bool f32 = false;
   int nx = 0, ny = 0, nz = 0;
+  int nf = 1;             // fields per transform: 3, or 1 where the slabs are padded
   long fs = 0;
-  void* spec = nullptr;   // half spectra of one field, (nx/2+1)*ny*nz complex
+  void* spec = nullptr;   // half spectra of nf fields, (nx/2+1)*ny*nz complex each
   void* rates = nullptr;  // (nx/2+1)*ny, element type
   void* term = nullptr;   // 3 slabs of fs: the terms of vx, vy, vz
 };
@@ -58,10 +59,11 @@ DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* r
   d->ny = ny;
   d->nz = nz;
   d->fs = fs;
+  d->nf = fs == (long)nx * ny * nz ? 3 : 1;
   const int mx = nx / 2 + 1;
   const long m = (long)mx * ny;
   const size_t esz = f32 ? sizeof(float) : sizeof(double);
-  bool ok = hipMalloc(&d->spec, 2 * esz * m * nz) == hipSuccess &&
+  bool ok = hipMalloc(&d->spec, 2 * esz * m * nz * d->nf) == hipSuccess &&
             hipMalloc(&d->rates, esz * m) == hipSuccess &&
             hipMalloc(&d->term, esz * 3 * fs) == hipSuccess;
   if (ok) {
@@ -73,12 +75,12 @@ DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* r
     }
   }
   // n, embeddings in C order (slowest first): a plane is ny rows of nx reals
-  // or of nx/2+1 complex values; batch = the nz planes of one field
+  // or of nx/2+1 complex values; batch = the nz planes of each field
   int n[2] = {ny, nx}, real_embed[2] = {ny, nx}, cplx_embed[2] = {ny, mx};
   ok = ok && hipfftPlanMany(&d->fwd, 2, n, real_embed, 1, nx * ny, cplx_embed, 1, (int)m,
-                            f32 ? HIPFFT_R2C : HIPFFT_D2Z, nz) == HIPFFT_SUCCESS;
+                            f32 ? HIPFFT_R2C : HIPFFT_D2Z, nz * d->nf) == HIPFFT_SUCCESS;
   ok = ok && hipfftPlanMany(&d->inv, 2, n, cplx_embed, 1, (int)m, real_embed, 1, nx * ny,
-                            f32 ? HIPFFT_C2R : HIPFFT_Z2D, nz) == HIPFFT_SUCCESS;
+                            f32 ? HIPFFT_C2R : HIPFFT_Z2D, nz * d->nf) == HIPFFT_SUCCESS;
   ok = ok && hipfftSetStream(d->fwd, st) == HIPFFT_SUCCESS && hipfftSetStream(d->inv, st) == HIPFFT_SUCCESS;
   if (!ok) {
     damp_destroy(d);
@@ -97,8 +99,8 @@ hipError_t damp_terms(DampPlan* d, const void* u, hipStream_t st) {
   const int mx = d->nx / 2 + 1;
   const int m = mx * d->ny;
   const size_t esz = d->f32 ? sizeof(float) : sizeof(double);
-  dim3 grid((unsigned)((m + 255) / 256), (unsigned)d->nz);
-  for (int f = 0; f < 3; ++f) {
+  dim3 grid((unsigned)((m + 255) / 256), (unsigned)(d->nz * d->nf));
+  for (int f = 0; f < 3; f += d->nf) {
     const char* in = (const char*)u + (size_t)(VX + f) * d->fs * esz;
     char* out = (char*)d->term + (size_t)f * d->fs * esz;
     hipfftResult r;
