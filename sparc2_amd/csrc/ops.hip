@@ -94,14 +94,20 @@ __global__ __launch_bounds__(256) void k_filter(const T* __restrict__ in, T* __r
 // y filter, then x filter of its result, each with its edge smoothing, one
 // read and one write per value.  A wave owns 64 consecutive x points (one per
 // lane, so loads and stores are coalesced) of one row segment and marches up
-// a chunk of KY rows with a register queue of the raw rows j-H .. j+H, loaded
-// PD rows ahead: the y stencil is read from registers.  The x stencil of the
-// y-filtered row is read from the neighbouring lanes (wavefront shuffles), so
-// the inner 64 - 2H lanes write results; the outer H lanes on each side only
-// supply the stencil (H = G + 1: the filter's reach plus the one-point reach
-// of the smoothing).  The per-point arithmetic is that of the separate passes,
-// in the same order, so both give the same bits.
-constexpr int FXY_KY = 64;
+// a chunk of ky rows.  The raw rows j-H .. j+H, and the PD rows loaded ahead of
+// them, sit in a ring of registers whose slots turn with the rows: the loop is
+// unrolled over one turn, so no value is moved.  The x stencil of the
+// y-filtered row is read from the neighbouring lanes by whole-wave shifts
+// (DPP, one vector move per shift and word, where a shuffle through LDS took a
+// round trip each), so the inner 64 - 2H lanes write results; the outer H
+// lanes on each side only supply the stencil (H = G + 1: the filter's reach
+// plus the one-point reach of the smoothing).  Rows whose stencil meets no
+// smoothed row take the plain sum.  The per-point arithmetic is that of the
+// separate passes, in the same order, so both give the same bits.
+// Bound by the vector instructions in FP32 and on the compensation terms, by
+// memory in FP64.  Five 384x384x160 fields: FP64 729 -> 450 us (1.89 GB), FP32
+// with its compensation 800 -> 575 (1.42 GB); eight of 63x79x101, 7 points,
+// FP64: 61 -> 24.
 constexpr int FXY_PD = 4;
 
 // S: the stored type -- T, or uint16_t for the FP32 form's bfloat16
@@ -115,17 +121,30 @@ template <typename T, typename S> __device__ __forceinline__ S to_s(T v) {
   else return v;
 }
 
+// The value of the lane below (UP) or above; 0 at the wave's end.
+template <bool UP> __device__ __forceinline__ int lane_next(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, UP ? 0x138 : 0x130, 0xF, 0xF, true);  // wave_shr:1, wave_shl:1
+}
+template <bool UP> __device__ __forceinline__ float lane_next(float v) {
+  return __builtin_bit_cast(float, lane_next<UP>(__builtin_bit_cast(int, v)));
+}
+template <bool UP> __device__ __forceinline__ double lane_next(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const unsigned lo = (unsigned)lane_next<UP>((int)(b & 0xFFFFFFFFll)), hi = (unsigned)lane_next<UP>((int)(b >> 32));
+  return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+
 template <typename T, int G, typename S = T>
 __global__ __launch_bounds__(256) void k_filter_xy(const S* __restrict__ in, S* __restrict__ out,
                                                    int nx, int ny, int nz, long fs, int nseg, int nych,
-                                                   long nwave, int periodic, T s,
+                                                   int ky, long nwave, int periodic, T s,
                                                    const int* __restrict__ halt) {
-  constexpr int H = G + 1, OW = 64 - 2 * H, Q = 2 * H + 1;
+  constexpr int H = G + 1, OW = 64 - 2 * H, R = 2 * H + 1 + FXY_PD;
   const int nblk = gridDim.x, b = blockIdx.x;
   const int xcd = b & 7, loc = b >> 3, base = nblk >> 3, rem = nblk & 7;
   const long lg = xcd * base + (xcd < rem ? xcd : rem) + loc;
-  const long wv = lg * 4 + (threadIdx.x >> 6);
-  if (wv >= nwave) return;  // whole waves only: the shuffles below see full waves
+  const long wv = lg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wv >= nwave) return;  // whole waves only: the shifts below see full waves
   const int lane = threadIdx.x & 63;
   const int seg = (int)(wv % nseg);
   long rest = wv / nseg;
@@ -135,10 +154,10 @@ __global__ __launch_bounds__(256) void k_filter_xy(const S* __restrict__ in, S* 
   const int f = (int)(rest / nz);
   const int x0 = seg * OW;
   const int xl = x0 - H + lane;  // this lane's x (unwrapped)
-  const bool xin = periodic || (xl >= 0 && xl < nx);
   const int xg = periodic ? wrap(xl, nx) : xl;
+  const bool xin = xg >= 0 && xg < nx;
   const bool writer = lane >= H && lane < 64 - H && xl < nx;
-  const int j0 = ych * FXY_KY, j1 = min(j0 + FXY_KY, ny);
+  const int j0 = ych * ky, j1 = min(j0 + ky, ny);
   const long plane = (long)f * fs + (long)nx * ny * k;
   const S* col = in + plane + (xin ? xg : 0);
   S* ocol = out + plane + xl;
@@ -148,119 +167,162 @@ __global__ __launch_bounds__(256) void k_filter_xy(const S* __restrict__ in, S* 
     return;
   }
   auto ld = [&](int r) -> T {
-    if (periodic) return (T)from_s(col[(long)wrap(r, ny) * nx]);
+    if (periodic) r = wrap1(r, ny);
     return (xin && r >= 0 && r < ny) ? (T)from_s(col[(long)r * nx]) : T(0);
   };
-  T q[Q], pf[FXY_PD];
+  // row j+d of the chunk's u-th row sits in slot (u + d + H) mod R
+  T q[R];
 #pragma unroll
-  for (int m = 0; m < Q - 1; ++m) q[m] = ld(j0 - H + m);
-#pragma unroll
-  for (int d = 0; d < FXY_PD; ++d) pf[d] = ld(j0 + H + d);
+  for (int m = 0; m < R - 1; ++m) q[m] = ld(j0 - H + m);
   const bool xedge = !periodic && ((xl >= 1 && xl <= G - 1) || (xl >= nx - G && xl <= nx - 2));
   const bool xcopy = !periodic && (xl < G || xl >= nx - G);
-  for (int j = j0; j < j1; ++j) {
-    q[Q - 1] = pf[0];
+  const bool xside = !periodic && (x0 - H < G || x0 - H + 63 >= nx - G);  // the wave meets such a point
+  for (int jb = j0; jb < j1; jb += R) {
 #pragma unroll
-    for (int d = 0; d < FXY_PD - 1; ++d) pf[d] = pf[d + 1];
-    pf[FXY_PD - 1] = ld(j + H + FXY_PD);
-    // y pass: smoothed raw value of row j+d (derivatives.f90:671-675)
-    auto smy = [&](int d) -> T {
-      const int r = j + d;
-      if (!periodic && ((r >= 1 && r <= G - 1) || (r >= ny - G && r <= ny - 2)))
-        return (q[d + H - 1] + q[d + H + 1]) / T(2);
-      return q[d + H];
-    };
-    T yf, y;
-    if (periodic) {
+    for (int u = 0; u < R; ++u) {
+      const int j = jb + u;
+      if (j >= j1) return;
+      q[(u + R - 1) % R] = ld(j + H + FXY_PD);
+      auto raw = [&](int d) -> T { return q[(u + d + H) % R]; };
+      // y pass: smoothed raw value of row j+d (derivatives.f90:671-675)
+      auto smy = [&](int d) -> T {
+        const int r = j + d;
+        if ((r >= 1 && r <= G - 1) || (r >= ny - G && r <= ny - 2)) return (raw(d - 1) + raw(d + 1)) / T(2);
+        return raw(d);
+      };
+      T yf, y;
+      if (periodic || (j >= 2 * G && j < ny - 2 * G)) {
+        T acc = 0;
+#pragma unroll
+        for (int m = -G; m <= G; ++m) acc += raw(m) * filt_w<T>(G, m);
+        yf = acc;
+        y = G == 5 ? yf : raw(0) - s * yf;
+      } else if (j < G || j >= ny - G) {
+        yf = G == 5 ? smy(0) : T(0);  // copy (g = 5) or zero (g = 3)
+        y = G == 5 ? yf : smy(0) - s * yf;
+      } else {
+        T acc = 0;
+#pragma unroll
+        for (int m = -G; m <= G; ++m) acc += smy(m) * filt_w<T>(G, m);
+        yf = acc;
+        y = G == 5 ? yf : smy(0) - s * yf;
+      }
+      // x pass on the y-filtered row across the lanes (derivatives.f90:680-687)
+      T sx = y;
+      if (xside) {
+        const T ym = lane_next<true>(y), yp = lane_next<false>(y);
+        sx = xedge ? (ym + yp) / T(2) : y;
+      }
+      T w[2 * G + 1];
+      w[G] = sx;
+#pragma unroll
+      for (int m = 1; m <= G; ++m) {
+        w[G - m] = lane_next<true>(w[G - m + 1]);
+        w[G + m] = lane_next<false>(w[G + m - 1]);
+      }
       T acc = 0;
 #pragma unroll
-      for (int m = -G; m <= G; ++m) acc += q[m + H] * filt_w<T>(G, m);
-      yf = acc;
-      y = G == 5 ? yf : q[H] - s * yf;
-    } else if (j < G || j >= ny - G) {
-      yf = G == 5 ? smy(0) : T(0);  // copy (g = 5) or zero (g = 3)
-      y = G == 5 ? yf : smy(0) - s * yf;
-    } else {
-      T acc = 0;
-#pragma unroll
-      for (int m = -G; m <= G; ++m) acc += smy(m) * filt_w<T>(G, m);
-      yf = acc;
-      y = G == 5 ? yf : smy(0) - s * yf;
+      for (int m = -G; m <= G; ++m) acc += w[G + m] * filt_w<T>(G, m);
+      T xf = acc;
+      if (xcopy) xf = G == 5 ? sx : T(0);
+      if (writer) ocol[(long)j * nx] = to_s<T, S>(G == 5 ? xf : sx - s * xf);
     }
-    // x pass on the y-filtered row across the lanes (derivatives.f90:680-687)
-    const T ym = __shfl_up(y, 1), yp = __shfl_down(y, 1);
-    const T sx = xedge ? (ym + yp) / T(2) : y;
-    T acc = 0;
-#pragma unroll
-    for (int m = -G; m <= G; ++m) {
-      const T v = m < 0 ? __shfl_up(sx, -m) : (m > 0 ? __shfl_down(sx, m) : sx);
-      acc += v * filt_w<T>(G, m);
-    }
-    T xf = acc;
-    if (xcopy) xf = G == 5 ? sx : T(0);
-    if (writer) ocol[(long)j * nx] = to_s<T, S>(G == 5 ? xf : sx - s * xf);
-#pragma unroll
-    for (int m = 0; m < Q - 1; ++m) q[m] = q[m + 1];
   }
 }
 
-// z filter: one column per thread marching up a chunk of planes with a
-// register queue of the raw values (planes pos-G-1 .. pos+G+1: the filter
-// reads smoothed values at pos-G .. pos+G, and a smoothed value reads its two
-// neighbours), so each value is loaded once; loads run ZPD planes ahead.
-// Same per-point arithmetic, in the same order, as k_filter along z.
+// z filter: CP adjacent columns per thread (2 in FP32, where the planes hold an
+// even number of points, so a lane's loads move 8 bytes) marching up a chunk of
+// planes with the raw planes pos-G-1 .. pos+G+1 and the ZPD planes loaded ahead
+// in a ring of registers, as above (the filter reads smoothed values at
+// pos-G .. pos+G, and a smoothed value reads its two neighbours), so each value
+// is loaded once.  Same per-point arithmetic, in the same order, as k_filter
+// along z.  Five 384x384x160 fields: FP64 498 -> 385 us (1.89 GB), FP32 with
+// its compensation 884 -> 348 (1.42 GB; moving the window took as many
+// instructions as the sum).
 constexpr int ZPD = 4;
 
-template <typename T, int G, typename S = T>
+template <typename T, int G, typename S, int CP>
 __global__ __launch_bounds__(256) void k_filter_z(const S* in, S* out,
                                                   int nx, int ny, int nz, long fs, int ncb, int kc,
                                                   T s, int bare, const int* __restrict__ halt) {
+  using V = typename Lane<T, CP>::V;
   const bool stop = halted(halt);  // guard stop: copy, as in k_filter
   const int nch = (nz + kc - 1) / kc;
   const int lg = blockIdx.x;
   const int cb = lg % ncb, rest = lg / ncb;
   const int chunk = rest % nch, f = rest / nch;
-  const long nxy = (long)nx * ny;
-  const long col = (long)cb * 256 + threadIdx.x;
+  const long nxy = (long)nx * ny;  // a multiple of CP
+  const long col = ((long)cb * 256 + threadIdx.x) * CP;
   if (col >= nxy) return;
   const S* line = in + (long)f * fs + col;
   S* o = out + (long)f * fs + col;
   const int k0 = chunk * kc, k1 = min(k0 + kc, nz);
   if (stop) {
-    for (int pos = k0; pos < k1; ++pos) o[(long)pos * nxy] = line[(long)pos * nxy];
+    for (int pos = k0; pos < k1; ++pos)
+      for (int c = 0; c < CP; ++c) o[(long)pos * nxy + c] = line[(long)pos * nxy + c];
     return;
   }
-  auto ld = [&](int r) -> T { return (r >= 0 && r < nz) ? (T)from_s(line[(long)r * nxy]) : T(0); };
-  constexpr int Q = 2 * G + 3;
-  T q[Q], pf[ZPD];
-#pragma unroll
-  for (int m = 0; m < Q - 1; ++m) q[m] = ld(k0 - G - 1 + m);
-#pragma unroll
-  for (int d = 0; d < ZPD; ++d) pf[d] = ld(k0 + G + 1 + d);
-  for (int pos = k0; pos < k1; ++pos) {
-    q[Q - 1] = pf[0];
-#pragma unroll
-    for (int d = 0; d < ZPD - 1; ++d) pf[d] = pf[d + 1];
-    pf[ZPD - 1] = ld(pos + G + 1 + ZPD);
-    // smoothed value of plane pos+d (derivatives.f90:690-693)
-    auto sm = [&](int d) -> T {
-      const int r = pos + d;
-      if (!bare && ((r >= 1 && r <= G - 1) || (r >= nz - G && r <= nz - 2)))
-        return (q[d + G] + q[d + G + 2]) / T(2);
-      return q[d + G + 1];
-    };
-    T filt;
-    if (pos < G || pos >= nz - G) {
-      filt = sm(0);  // z: copy for both widths (derivatives.f90:624,635)
+  auto ld = [&](int r) -> V {
+    if (r < 0 || r >= nz) return V(0);
+    const S* p = line + (long)r * nxy;
+    if constexpr (CP == 1) {
+      return (T)from_s(*p);
+    } else if constexpr (sizeof(S) == 2) {
+      const uint32_t u = *(const uint32_t*)p;
+      return V(bf2f((uint16_t)(u & 0xFFFFu)), bf2f((uint16_t)(u >> 16)));
     } else {
-      T acc = 0;
-#pragma unroll
-      for (int m = -G; m <= G; ++m) acc += sm(m) * filt_w<T>(G, m);
-      filt = acc;
+      const float2 u = *(const float2*)p;
+      return V(u.x, u.y);
     }
-    o[(long)pos * nxy] = to_s<T, S>((G == 5 || bare) ? filt : sm(0) - s * filt);
+  };
+  auto st = [&](int r, V v) {
+    S* p = o + (long)r * nxy;
+    if constexpr (CP == 1) {
+      *p = to_s<T, S>(v);
+    } else if constexpr (sizeof(S) == 2) {
+      *(uint32_t*)p = (uint32_t)f2bf(v.x) | ((uint32_t)f2bf(v.y) << 16);
+    } else {
+      *(float2*)p = make_float2(v.x, v.y);
+    }
+  };
+  constexpr int R = 2 * G + 3 + ZPD;
+  // plane pos+d of the chunk's u-th plane sits in slot (u + d + G + 1) mod R
+  V q[R];
 #pragma unroll
-    for (int m = 0; m < Q - 1; ++m) q[m] = q[m + 1];
+  for (int m = 0; m < R - 1; ++m) q[m] = ld(k0 - G - 1 + m);
+  for (int kb = k0; kb < k1; kb += R) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int pos = kb + u;
+      if (pos >= k1) return;
+      q[(u + R - 1) % R] = ld(pos + G + 1 + ZPD);
+      auto raw = [&](int d) -> V { return q[(u + d + G + 1) % R]; };
+      // smoothed value of plane pos+d (derivatives.f90:690-693)
+      auto sm = [&](int d) -> V {
+        const int r = pos + d;
+        if (!bare && ((r >= 1 && r <= G - 1) || (r >= nz - G && r <= nz - 2))) return (raw(d - 1) + raw(d + 1)) * V(T(0.5));
+        return raw(d);
+      };
+      V filt, centre;
+      if (pos >= 2 * G && pos < nz - 2 * G) {  // no smoothed plane in reach
+        V acc = 0;
+#pragma unroll
+        for (int m = -G; m <= G; ++m) acc += raw(m) * V(filt_w<T>(G, m));
+        filt = acc;
+        centre = raw(0);
+      } else {
+        centre = sm(0);
+        if (pos < G || pos >= nz - G) {
+          filt = centre;  // z: copy for both widths (derivatives.f90:624,635)
+        } else {
+          V acc = 0;
+#pragma unroll
+          for (int m = -G; m <= G; ++m) acc += sm(m) * V(filt_w<T>(G, m));
+          filt = acc;
+        }
+      }
+      st(pos, (G == 5 || bare) ? filt : centre - s * filt);
+    }
   }
 }
 
@@ -275,22 +337,34 @@ hipError_t launch_filter_zc(int g, const void* in, void* out, int nx, int ny, in
   if (cbf && sizeof(T) != 4) return hipErrorInvalidValue;
   // column blocks x z chunks x fields: >= ~2048 blocks, chunks >= 16 deep
   const long nxy = (long)nx * ny;
-  const int ncb = (int)((nxy + 255) / 256);
+  const int cp = sizeof(T) == 4 && nxy % 2 == 0 ? 2 : 1;
+  const int ncb = (int)((nxy + 256 * cp - 1) / (256 * cp));
   const long want = (2048 + (long)ncb * nfield - 1) / ((long)ncb * nfield);
   const int nch = inplace ? 1 : (int)std::max(1L, std::min(want, (long)nz / 16));
   const int kc = (nz + nch - 1) / nch;
   const long nb = (long)ncb * ((nz + kc - 1) / kc) * nfield;
   if (nb >= (1L << 31)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)nb);
-#define SPARC_FZ(GG, S) \
-  hipLaunchKernelGGL((k_filter_z<T, GG, S>), grid, dim3(256), 0, st, (const S*)in, (S*)out, nx, ny, nz, fs, ncb, kc, s, bare, halt)
-  if (cbf) {
-    if (g == 5) SPARC_FZ(5, uint16_t);
-    else SPARC_FZ(3, uint16_t);
+#define SPARC_FZ(GG, S, CP)                                                                           \
+  hipLaunchKernelGGL((k_filter_z<T, GG, S, CP>), grid, dim3(256), 0, st, (const S*)in, (S*)out, nx, ny, nz, fs, ncb, \
+                     kc, s, bare, halt)
+#define SPARC_FZG(S, CP) \
+  if (g == 5) SPARC_FZ(5, S, CP); \
+  else SPARC_FZ(3, S, CP)
+  if constexpr (sizeof(T) == 4) {
+    if (cbf && cp == 2) {
+      SPARC_FZG(uint16_t, 2);
+    } else if (cbf) {
+      SPARC_FZG(uint16_t, 1);
+    } else if (cp == 2) {
+      SPARC_FZG(T, 2);
+    } else {
+      SPARC_FZG(T, 1);
+    }
   } else {
-    if (g == 5) SPARC_FZ(5, T);
-    else SPARC_FZ(3, T);
+    SPARC_FZG(T, 1);
   }
+#undef SPARC_FZG
 #undef SPARC_FZ
   return hipGetLastError();
 }
@@ -304,7 +378,12 @@ template <typename T>
 hipError_t launch_filter_xy(int g, const void* in, void* out, int nx, int ny, int nz, long fs,
                             int nfield, int periodic, T s, hipStream_t st, const int* halt, bool cbf) {
   const int ow = 64 - 2 * (g + 1);
-  const int nseg = (nx + ow - 1) / ow, nych = (ny + FXY_KY - 1) / FXY_KY;
+  const int nseg = (nx + ow - 1) / ow;
+  // rows per wave: 64, or fewer where that leaves under 8192 waves (a chunk
+  // re-reads 2 (g + 1) rows, but a wave takes its rows one after the other)
+  int ky = 64;
+  while (ky > 16 && (long)nseg * ((ny + ky - 1) / ky) * nz * nfield < 8192) ky /= 2;
+  const int nych = (ny + ky - 1) / ky;
   const long nwave = (long)nseg * nych * nz * nfield;
   const long nb = (nwave + 3) / 4;
   if (nb >= (1L << 31)) return hipErrorInvalidValue;
@@ -312,7 +391,7 @@ hipError_t launch_filter_xy(int g, const void* in, void* out, int nx, int ny, in
   const dim3 grid((unsigned)nb);
 #define SPARC_FXY(GG, S)                                                                              \
   hipLaunchKernelGGL((k_filter_xy<T, GG, S>), grid, dim3(256), 0, st, (const S*)in, (S*)out, nx, ny, \
-                     nz, fs, nseg, nych, nwave, periodic, s, halt)
+                     nz, fs, nseg, nych, ky, nwave, periodic, s, halt)
   if (cbf) {
     if (g == 5) SPARC_FXY(5, uint16_t);
     else SPARC_FXY(3, uint16_t);
