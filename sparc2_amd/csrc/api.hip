@@ -389,14 +389,23 @@ static void choose_tile(sparc_ctx* c) {
   const sparc_cfg& q = c->cfg;
   int tx = q.tile[0], ty = q.tile[1];
   if (!(tx > 0 && ty > 0 && stage_tile_supported(tx, ty))) {
+    // Grids whose rows are not whole 128-byte lines: a tile's row of 128 bytes
+    // (16 lanes of 8) then touches two lines and one of 256 bytes three, so
+    // the wider tile fetches a quarter less (MHD FP64 191x175x130, best chunk
+    // of each shape: 16x16 588 us, 32x8 492, 32x16 481; 150x90x120 233 / - /
+    // 201; quiet FP64 250x130x140 222 / 182 / 171).  Two-point FP32 MHD lanes
+    // stay at 16x16 (150x90x120: 113 us, 32x16 129).
+    const bool lines = (size_t)c->nx * c->esz % 128 == 0;
     static const int quiet64[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
+    static const int quiet64m[4][2] = {{32, 16}, {32, 8}, {16, 16}, {64, 4}};
     static const int quiet32[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
     static const int mhd64[4][2] = {{16, 16}, {32, 16}, {32, 8}, {64, 4}};
+    static const int mhd64m[4][2] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
     static const int mhd32[4][2] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
     // two points per lane (FP32, even nx): the MHD xy kernel at 16x16 lanes
     static const int mhd32x2[4][2] = {{16, 16}, {32, 8}, {32, 16}, {64, 4}};
-    const int(*pref)[2] = c->mhd ? (c->f32 ? (c->vw == 2 ? mhd32x2 : mhd32) : mhd64)
-                                 : (c->f32 ? quiet32 : quiet64);
+    const int(*pref)[2] = c->mhd ? (c->f32 ? (c->vw == 2 ? mhd32x2 : mhd32) : (lines ? mhd64 : mhd64m))
+                                 : (c->f32 ? quiet32 : (lines ? quiet64 : quiet64m));
     tx = 32;
     ty = 8;
     double least = 1e300;
@@ -405,9 +414,13 @@ static void choose_tile(sparc_ctx* c) {
       if (c->nx <= 16 && pref[n][0] * c->vw > 16) continue;
       if (!tile_fits(c, pref[n][0], pref[n][1])) continue;
       // the MHD shapes in order of preference; a quiet run takes the shape
-      // whose launch is shortest (auto_chunk), the preferred of equal ones
+      // whose launch is shortest (auto_chunk, with 15% for the second line of
+      // 128-byte rows), the preferred of equal ones
       double cost = 0.0;
-      if (!c->mhd) auto_chunk(c, pref[n][0], pref[n][1], &cost);
+      if (!c->mhd) {
+        auto_chunk(c, pref[n][0], pref[n][1], &cost);
+        if (!lines) cost *= 1.0 + 0.15 * 128.0 / (double)(pref[n][0] * c->vw * c->esz);
+      }
       if (cost < least) {
         least = cost;
         tx = pref[n][0];
@@ -455,19 +468,25 @@ static int balanced_chunk(long tiles, int nz, long places, double c0, int kmax, 
 //  quiet: the window re-reads 10 planes of two fields per chunk, and a start
 //    takes as long as 4 planes (fitted over 48x48x96 .. 512x512x300);
 //  quiet with x and y CPML: the tiles at the sides take longer than the inner
-//    ones, and chunks of at most 10 planes even that out (192x192x128 FP64
-//    350 us at 36 planes, 239 at 10);
-//  MHD xy kernel: no window, half a plane to start; at most 6 planes, so the
-//    halo rows are still in L2 when the neighbouring tiles read them (256^3
-//    FP64 1484 us at 4 planes, 1473 at 6, 1515 at 12; 64x128x160 FP32, where
-//    5 planes make one round of 512 blocks, 101 us at 4 and 78 at 5).
+//    ones, and chunks of at most 5 planes (10 in FP32, whose planes are
+//    shorter) even that out (192x192x128 FP64 350
+//    us at 36 planes, 227 at 9, 218 at 5; 107x75x117 32x16 81 at 10, 75 at 5);
+//  MHD xy kernel: no window, half a plane to start; at most 6 planes (5 in
+//    FP32), so the halo rows are still in L2 when the neighbouring tiles read
+//    them (256^3 FP64 1484 us at 4 planes, 1473 at 6, 1515 at 12; 64x128x160
+//    FP32, where 5 planes make one round of 512 blocks, 101 us at 4 and 78 at
+//    5), and at most 2 where the tiles' rows share lines with their neighbours
+//    too (191x175x130 FP64 32x8 492 us at 2 planes, 513 at 5; FP32 276 / 299).
 static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost) {
   const long tiles = (long)((c->nx + tx * c->vw - 1) / (tx * c->vw)) * ((c->ny + ty - 1) / ty);
   const bool dma = c->dma && tx == 16 && ty == 16;
   const int places = c->f32 ? stage_resident<float>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma)
                             : stage_resident<double>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma);
-  if (c->zp) return balanced_chunk(tiles, c->nz, places, 0.5, c->f32 ? 5 : 6, cost);
-  return balanced_chunk(tiles, c->nz, places, 4.0, c->cfg.use_hpml ? 10 : c->nz, cost);
+  if (c->zp) {
+    const bool lines = (size_t)c->nx * c->esz % 128 == 0;
+    return balanced_chunk(tiles, c->nz, places, 0.5, !lines ? 2 : (c->f32 ? 5 : 6), cost);
+  }
+  return balanced_chunk(tiles, c->nz, places, 4.0, !c->cfg.use_hpml ? c->nz : (c->f32 ? 10 : 5), cost);
 }
 
 // Tile shape, z chunk (kc <= 0: automatic) and the z pass's chunking.
