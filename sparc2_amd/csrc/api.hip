@@ -158,7 +158,7 @@ struct sparc_ctx {
   int guard_mode = GUARD_HALT;
   double dimc = 1.0, dimrho = 1.0;
   int tx = 64, ty = 8, kc = 8, ntx = 1, nty = 1, nchunk = 1;
-  int zkc = 8, znchunk = 1;  // z-pass chunking
+  int zn = 1;  // z-pass chunks
   bool kc_auto = true;       // kc follows auto_chunk
   int ncu = 256;
   bool bg_set = false, state_set = false;
@@ -501,14 +501,15 @@ static void set_geometry(sparc_ctx* c, int tx, int ty, int kc) {
   c->nchunk = (c->nz + kc - 1) / kc;
   // z pass: blocks of 256 columns, streaming, at full rate with half the
   // blocks that fit (one per CU in FP64, two in FP32); the 10-plane window a
-  // chunk reads first costs as much as 14 planes (fitted from 1 to 256 planes
-  // on eight grids: 63x79x101 FP64 55 us at 34 planes, 35 at 10; 256^3 FP64
-  // 423 at 128, 390 at 256, 473 at 64; 192x192x160 FP64 215 at 46, 187 at 64)
+  // chunk reads first costs as much as 14 planes.  The number of chunks this
+  // gives is the best of 1 .. 28, or within 3 %, on ten grids (63x79x101 FP64
+  // 12 chunks 26 us, 8 33, 13 35; 128x96x96 FP64 5 45, 3 57, 6 57; 256^3 FP64
+  // 1 375, 2 417; 192x192x160 FP32 3 87, 2 111, 5 85)
   if (c->zp) {
     const long ncb = ((long)c->nx * c->ny + 255) / 256;
     const int places = (c->f32 ? zpass_resident<float>(c->ncu) : zpass_resident<double>(c->ncu)) / 2;
-    c->zkc = balanced_chunk(ncb, c->nz, std::max(1, places), 14.0, c->nz, nullptr);
-    c->znchunk = (c->nz + c->zkc - 1) / c->zkc;
+    const int kc = balanced_chunk(ncb, c->nz, std::max(1, places), 14.0, c->nz, nullptr);
+    c->zn = (c->nz + kc - 1) / kc;
   }
 }
 
@@ -901,7 +902,7 @@ static void fill_common(sparc_ctx* c, StageArgs<T>& A) {
   A.fs = c->fs;
   A.ntx = c->ntx;
   A.nblk_xy = c->ntx * c->nty;
-  A.zkc = c->zkc;
+  A.zn = c->zn;
   auto lo = [&](int f) { return c->face[f].active ? c->face[f].n : 0; };
   auto hi = [&](int f, int n) { return c->face[f].active ? c->face[f].off : n; };
   A.xlo = lo(XBOT);
@@ -1002,7 +1003,7 @@ static GuardArgs guard_args(const sparc_ctx* c) {
 
 template <typename T>
 static hipError_t enqueue_zpass(sparc_ctx* c, const StageArgs<T>& A) {
-  return launch_zpass<T>(A, zpass_items(c->nx, c->ny, c->znchunk), c->st);
+  return launch_zpass<T>(A, zpass_items(c->nx, c->ny, c->zn), c->st);
 }
 template <typename T>
 static hipError_t enqueue_stage(sparc_ctx* c, const StageArgs<T>& A, double amp) {
@@ -1389,7 +1390,7 @@ struct BatchGroup {
   int vw = 1, tx = 0, ty = 0, nblk = 0, znblk = 0;
   std::vector<int> members;
   std::vector<int> kc;         // z chunk depth per member in this batch
-  std::vector<int> zkc;        // z-pass chunk depth per member in this batch
+  std::vector<int> zn;         // z-pass chunks per member in this batch
   void* args[5] = {};         // StageArgs<T>[members] per stage (device)
   int* item_start = nullptr;   // prefix of stage work items (device)
   int* zitem_start = nullptr;  // prefix of z-pass work items (device)
@@ -1441,7 +1442,7 @@ static int batch_upload_args(sparc_batch* b) {
         fill_common<T>(c, h[q]);
         set_stage<T>(c, h[q], s);
         h[q].kc = g.kc[q];
-        if (g.zp) h[q].zkc = g.zkc[q];
+        if (g.zp) h[q].zn = g.zn[q];
         h[q].amp_tab = c->cfg.pulse_dir ? (const T*)b->amp[r] : nullptr;
         h[q].tstep = b->tstep;
       }
@@ -1594,12 +1595,12 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
       for (int r : g.members) ncols += zpass_items(b->runs[r]->nx, b->runs[r]->ny, 1);
       const long per_run = std::max<long>(1, (2L * g.znblk + ncols - 1) / ncols);
       std::vector<int> zs(g.members.size() + 1, 0);
-      g.zkc.assign(g.members.size(), 0);
+      g.zn.assign(g.members.size(), 1);
       for (size_t q = 0; q < g.members.size(); ++q) {
         const sparc_ctx* c = b->runs[g.members[q]];
         const int kc = (int)std::min<long>(c->nz, std::max<long>(48, (c->nz + per_run - 1) / per_run));
-        g.zkc[q] = kc;
-        zs[q + 1] = zs[q] + (int)zpass_items(c->nx, c->ny, (c->nz + kc - 1) / kc);
+        g.zn[q] = (c->nz + kc - 1) / kc;
+        zs[q + 1] = zs[q] + (int)zpass_items(c->nx, c->ny, g.zn[q]);
       }
       if ((rc = dalloc((void**)&g.zitem_start, sizeof(int) * zs.size()))) return bail(rc);
       if (hipMemcpy(g.zitem_start, zs.data(), sizeof(int) * zs.size(), hipMemcpyHostToDevice) != hipSuccess)

@@ -157,7 +157,7 @@ template <typename T> struct StageArgs {
   // FP64 MHD xy kernel divides (correctly rounded, the same bits) instead of
   // reading the array
   int rinv_rho0;
-  int zkc;  // MHD z pass: its own z chunk (deeper: the queue warm-up re-reads 10 planes)
+  int zn;  // MHD z pass: its own z chunks (fewer: the queue warm-up re-reads 10 planes)
   const T* stretch_lo;  // nz remainders of stretch(k) (FP32 only)
   // batches: the source amplitude is amp_tab[*tstep] (a device table and step
   // counter, so a captured step replays unchanged); a single run's comes with
@@ -497,6 +497,21 @@ __device__ __forceinline__ void pml_face(FR& F, uint32_t fp, V (&v)[NF], const i
     else
       stv<CPW>(Buf<T>(F.pst + (size_t)fam[i] * n, n), fp, base[i] + beta_next * kn);
   }
+}
+
+// First plane of chunk c of the z pass's n chunks (c = n: nz).  Chunks take
+// equal shares of the work rather than of the planes: a plane inside a z-face
+// layer counts ZCUT_FACE, one between them ZCUT_INNER (36 arrays are read or
+// written there against 15), so that the first and the last chunk are not
+// what the others wait for (z pass 63x79x101 FP64 32.3 -> 26.3 us, FP32 22.8
+// -> 20.9, 64x128x160 FP32 35.5 -> 28.2; a grid of one chunk stays as it is).
+constexpr int ZCUT_INNER = 2, ZCUT_FACE = 5;
+__device__ __forceinline__ int zpass_cut(int c, int n, int zlo, int zhi, int nz) {
+  const int bot = min(zlo, nz), mid = max(0, min(zhi, nz) - bot), top = nz - bot - mid;
+  const int t = (int)((long)c * (ZCUT_FACE * (bot + top) + ZCUT_INNER * mid) / n);
+  if (t < ZCUT_FACE * bot) return t / ZCUT_FACE;
+  if (t < ZCUT_FACE * bot + ZCUT_INNER * mid) return bot + (t - ZCUT_FACE * bot) / ZCUT_INNER;
+  return bot + mid + (t - ZCUT_FACE * bot - ZCUT_INNER * mid) / ZCUT_FACE;
 }
 
 // One period to either side, without a division: an index that is still
