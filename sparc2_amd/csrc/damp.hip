@@ -26,11 +26,11 @@ namespace sparc {
 // Through the library a plane passes five launches (x and y transforms each
 // way, the multiply) that read and write it ten times.  Here one block reads it
 // once and writes the term once.  Three velocities, all planes, FP64: 48x48x96
-// 39 -> 19 us, 64x96x100 61 -> 32, 100x100x100 136 -> 60, 128x128x64 65 -> 41,
-// 128x96x100 81 -> 68 (100 KB, so one block a CU, and 300 blocks are two rounds
-// of 256), 75x75x300 297 -> 70; FP32 128x128x128 78 -> 39, 160x120x100 118 -> 42.
-// What is left is LDS traffic: a pass moves the plane at about 54 bytes a clock
-// and CU, and two of nine passes' worth of time goes to the first load.
+// 39 -> 17 us, 64x96x100 61 -> 30, 100x100x100 136 -> 48, 128x128x64 65 -> 36,
+// 128x96x100 81 -> 56 (100 KB, so one block a CU, and 300 blocks are two rounds
+// of 256), 75x75x300 297 -> 67; FP32 128x96x100 67 -> 31, 128x128x128 78 -> 36.
+// What bounds it: the first load, at the rate of HBM, then the LDS passes, each
+// a round trip of the plane and the fetch of its instructions.
 //
 // Two rows r and r + ny/2 travel as the real and imaginary part of one complex
 // line through the x transform, so LDS holds the plane's half spectrum (64x96
@@ -41,10 +41,10 @@ namespace sparc {
 // pass of the way in and the first of the way back hold the same values:
 // transform, multiply and transform back happen in registers.  The outer y
 // passes hold both rows of a line where their radix is even, and split and join
-// them.  The fewest passes win, up to radix 16 (128x96x100: radices up to 16 68
-// us, up to 12 75, up to 8 79, up to 4 92).  Lanes run over the lines and the
-// line stride S is odd, so x passes are free of bank conflicts; y passes take
-// the columns in the order in which they lie.
+// them.  The fewest passes win, up to radix 16 (128x96x100: radices up to 16 56
+// us, up to 12 61, up to 8 67).  Lanes run over the lines and the line stride S
+// is odd, so x passes are free of bank conflicts; y passes take the columns in
+// the order in which they lie.
 // ---------------------------------------------------------------------------
 constexpr int DP_MAXPASS = 8;
 constexpr size_t kLdsBytes = 160 * 1024;
@@ -203,32 +203,33 @@ template <typename T> __device__ __forceinline__ void join_rows(Cx<T>& a, Cx<T>&
   b = w;  // own: never read again
 }
 
-// One pass of radix R over all lines of length n, blocks of R * m.  Y: along
-// the columns; RATE: the last pass of the way in and the first of the way back
-// (m = 1, no twiddles) with the multiply between them; ends: see DampShape.  A
-// wave takes one butterfly of 64 lines, so its indices are scalars; up to
-// kSpare lines that are left over (a power of two has 2^k + 1 columns) share
-// waves, lanes over lines and butterflies (48x48x96, 24 and 25 lines: 22 us
-// shared, 25 with most lanes idle; 100x100 and up the same).
-constexpr int kSpare = 40;
-template <int NT, int R, bool Y, bool INV, bool RATE, typename T>
+// One pass of radix R over all lines of length n along x, or along the columns
+// (y), in blocks of R * m.  WAY: in, back, or the last pass of the way in and
+// the first of the way back (m = 1, no twiddles) with the multiply between
+// them; ends: see DampShape.  Lanes run over lines first, then butterflies.
+// One code serves x and y and all lines: a block runs through some 70 KB of
+// instructions once or twice otherwise, and what it waited for was their fetch
+// (a second code with scalar indices for whole waves of lines, and x and y
+// apart: 128x96x100 68 us, 100x100x100 60).
+enum Way { IN, BACK, RATES };
+template <int NT, int R, int WAY, typename T>
 __device__ __forceinline__ void damp_pass(const DampShape& D, Cx<T>* __restrict__ L, const Cx<T>* __restrict__ tw,
-                                          const ushort2* __restrict__ cols, const T* __restrict__ rates, int m,
+                                          const ushort2* __restrict__ cols, const T* __restrict__ rates, int m, bool y,
                                           bool ends) {
-  const int n = Y ? D.ny : D.nx, nl = Y ? D.mx : D.pairs, nb = n / R;
+  const int n = y ? D.ny : D.nx, nl = y ? D.mx : D.pairs, nb = n / R;
   const int step = nb / m;  // blocks; w_{R m} = w_n^step
-  const Divide by_m(m);
-  auto butterfly = [&](int line, int b) {
-    const int g = by_m(b), j = b - g * m, e0 = g * R * m + j;
-    const int ca = Y ? cols[line].x : line * D.S, cb = Y ? cols[line].y - D.pairs * D.S : 0;
-    auto at = [&](int r) {
-      const int e = e0 + r * m;
-      return Y ? e * D.S + (e < D.pairs ? ca : cb) : ca + e;
-    };
+  const int es = y ? D.S : 1, ms = m * es, half = y ? D.pairs : n;
+  const Divide by_line(nl), by_m(m);
+  for (int t = (int)threadIdx.x; t < nl * nb; t += NT) {
+    const int b = by_line(t), line = t - b * nl, g = by_m(b), j = b - g * m, e0 = g * R * m + j;
+    const ushort2 col = cols[y ? line : 0];
+    const int ca = (y ? col.x : line * D.S) + e0 * es, cb = ca - col.x + col.y - D.pairs * D.S;
+    auto at = [&](int r) { return (e0 + r * m < half ? ca : cb) + r * ms; };
     Cx<T> v[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = L[at(r)];
-    if constexpr (RATE) {
+    const bool own = col.y >= D.nx;
+    if constexpr (WAY == RATES) {
       T w[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) w[q] = rates[(e0 + q) * nl + line];
@@ -238,18 +239,17 @@ __device__ __forceinline__ void damp_pass(const DampShape& D, Cx<T>* __restrict_
       dft<R, true>(v);
     } else {
       const int js = j * step;
-      const bool own = Y && cols[line].y >= D.nx;
-      if constexpr (Y && !INV && R % 2 == 0) {
+      if constexpr (WAY == IN && R % 2 == 0) {
         if (ends) {
 #pragma unroll
           for (int r = 0; r < R / 2; ++r) split_rows(v[r], v[r + R / 2], own);
         }
       }
-      if constexpr (!INV) dft<R, false>(v);
+      if constexpr (WAY == IN) dft<R, false>(v);
 #pragma unroll
-      for (int q = 1; q < R; ++q) v[q] = turn<INV>(v[q], tw[js * q]);
-      if constexpr (INV) dft<R, true>(v);
-      if constexpr (Y && INV && R % 2 == 0) {
+      for (int q = 1; q < R; ++q) v[q] = turn<WAY == BACK>(v[q], tw[js * q]);
+      if constexpr (WAY == BACK) dft<R, true>(v);
+      if constexpr (WAY == BACK && R % 2 == 0) {
         if (ends) {
 #pragma unroll
           for (int r = 0; r < R / 2; ++r) join_rows(v[r], v[r + R / 2], own);
@@ -258,38 +258,24 @@ __device__ __forceinline__ void damp_pass(const DampShape& D, Cx<T>* __restrict_
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) L[at(r)] = v[r];
-  };
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
-  const int rest = nl & 63, whole = rest <= kSpare ? nl - rest : nl;
-  for (int l0 = 0; l0 < whole; l0 += 64) {
-    const int line = l0 + lane;
-    if (line < nl)
-      for (int b = wave; b < nb; b += NT / 64) butterfly(line, b);
-  }
-  if (whole < nl) {
-    const Divide by_rest(rest);
-    for (int t = NT - 1 - (int)threadIdx.x; t < rest * nb; t += NT) {
-      const int b = by_rest(t);
-      butterfly(whole + t - b * rest, b);
-    }
   }
   __syncthreads();
 }
 
-template <int NT, bool Y, bool INV, bool RATE, typename T>
+template <int NT, int WAY, typename T>
 __device__ __forceinline__ void damp_radix(const DampShape& D, int R, Cx<T>* L, const Cx<T>* tw, const ushort2* cols,
-                                           const T* rates, int m, bool ends = false) {
+                                           const T* rates, int m, bool y, bool ends = false) {
   switch (R) {
-    case 2: damp_pass<NT, 2, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 3: damp_pass<NT, 3, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 4: damp_pass<NT, 4, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 5: damp_pass<NT, 5, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 6: damp_pass<NT, 6, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 7: damp_pass<NT, 7, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 8: damp_pass<NT, 8, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 10: damp_pass<NT, 10, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    case 12: damp_pass<NT, 12, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
-    default: damp_pass<NT, 16, Y, INV, RATE>(D, L, tw, cols, rates, m, ends); break;
+    case 2: damp_pass<NT, 2, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 3: damp_pass<NT, 3, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 4: damp_pass<NT, 4, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 5: damp_pass<NT, 5, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 6: damp_pass<NT, 6, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 7: damp_pass<NT, 7, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 8: damp_pass<NT, 8, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 10: damp_pass<NT, 10, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    case 12: damp_pass<NT, 12, WAY>(D, L, tw, cols, rates, m, y, ends); break;
+    default: damp_pass<NT, 16, WAY>(D, L, tw, cols, rates, m, y, ends); break;
   }
 }
 
@@ -333,11 +319,6 @@ __global__ __launch_bounds__(NT, 4) void k_damp_plane(const DampShape D, const T
   for (int t = tid; t < D.mx; t += NT) cols[t] = places[t];
   __syncthreads();
 
-  int m = nx;
-  for (int p = 0; p < D.npx; ++p) {
-    m /= D.rx[p];
-    damp_radix<NT, false, false, false>(D, D.rx[p], L, twx, cols, rates, m);
-  }
   // f on the two values of every column in every line
   auto each_column = [&](auto f) {
     for (int t = tid; t < D.pairs * D.mx; t += NT) {
@@ -350,23 +331,30 @@ __global__ __launch_bounds__(NT, 4) void k_damp_plane(const DampShape D, const T
     }
     __syncthreads();
   };
-  if (!D.ends) each_column([](Cx<T>& z, Cx<T>& w, bool own) { split_rows(z, w, own); });
-  m = ny;
-  for (int p = 0; p + 1 < D.npy; ++p) {
-    m /= D.ry[p];
-    damp_radix<NT, true, false, false>(D, D.ry[p], L, twy, cols, rates, m, D.ends && p == 0);
+  // the way in: the x passes, the rows apart, the y passes but one
+  for (int p = 0, m = nx; p < D.npx + D.npy - 1; ++p) {
+    const bool y = p >= D.npx;
+    if (p == D.npx) {
+      m = ny;
+      if (!D.ends) each_column([](Cx<T>& z, Cx<T>& w, bool own) { split_rows(z, w, own); });
+    }
+    const int R = y ? D.ry[p - D.npx] : D.rx[p];
+    m /= R;
+    damp_radix<NT, IN>(D, R, L, y ? twy : twx, cols, rates, m, y, p == D.npx && D.ends);
   }
-  damp_radix<NT, true, false, true>(D, D.ry[D.npy - 1], L, twy, cols, rates, 1);
-  m = D.ry[D.npy - 1];
-  for (int p = D.npy - 2; p >= 0; --p) {
-    damp_radix<NT, true, true, false>(D, D.ry[p], L, twy, cols, rates, m, D.ends && p == 0);
-    m *= D.ry[p];
-  }
-  if (!D.ends) each_column([](Cx<T>& a, Cx<T>& b, bool own) { join_rows(a, b, own); });
-  m = 1;
-  for (int p = D.npx - 1; p >= 0; --p) {
-    damp_radix<NT, false, true, false>(D, D.rx[p], L, twx, cols, rates, m);
-    m *= D.rx[p];
+  if (D.npy == 1) each_column([](Cx<T>& z, Cx<T>& w, bool own) { split_rows(z, w, own); });
+  damp_radix<NT, RATES>(D, D.ry[D.npy - 1], L, twy, cols, rates, 1, true);
+  if (D.npy == 1) each_column([](Cx<T>& a, Cx<T>& b, bool own) { join_rows(a, b, own); });
+  // and back
+  for (int p = D.npx + D.npy - 2, m = D.npy > 1 ? D.ry[D.npy - 1] : 1; p >= 0; --p) {
+    const bool y = p >= D.npx;
+    const int R = y ? D.ry[p - D.npx] : D.rx[p];
+    damp_radix<NT, BACK>(D, R, L, y ? twy : twx, cols, rates, m, y, p == D.npx && D.ends);
+    m *= R;
+    if (p == D.npx) {
+      m = 1;
+      if (!D.ends) each_column([](Cx<T>& a, Cx<T>& b, bool own) { join_rows(a, b, own); });
+    }
   }
   for (int t = tid; t < cells; t += NT) {
     const int r = by_nx(t), x = t - r * nx;
@@ -463,16 +451,15 @@ static bool plane_shape(DampPlan* d) {
   return D.npx > 0 && D.npy > 0 && d->lds <= kLdsBytes;
 }
 
-// Threads of a block: enough for a CU's SIMDs together with the blocks that
-// share it.  64x96x100 FP64 (three blocks a CU) 35 us with 256, 32 with 512, 42
-// with 1024; 48x48x200 (eight) 25 with 256, 37 with 512; 60x60x200 (five) 30 /
-// 43, 64x64x64 (four) 22 / 21; 128x128x64 (one) 47 with 512, 43 with 1024.
-static int plane_threads(const DampPlan* d) { return 5 * d->lds <= kLdsBytes ? 256 : (2 * d->lds <= kLdsBytes ? 512 : 1024); }
+// Threads of a block: 256 where five or more share a CU, which then fill its
+// SIMDs together (60x60x200 FP64 29 us, 34 with 512), else 512 (64x64x64, four
+// a CU, 18 us, 19 with 256; 128x96x100, one a CU, 56, 69 with 256; 1024 no
+// faster there).
+static int plane_threads(const DampPlan* d) { return 5 * d->lds <= kLdsBytes ? 256 : 512; }
 
 template <typename T> using PlaneKernel = void (*)(const DampShape, const T*, T*, const Cx<T>*, const ushort2*, const T*);
 template <typename T> static PlaneKernel<T> plane_kernel(const DampPlan* d) {
-  const int nt = plane_threads(d);
-  return nt == 256 ? k_damp_plane<T, 256> : (nt == 512 ? k_damp_plane<T, 512> : k_damp_plane<T, 1024>);
+  return plane_threads(d) == 256 ? k_damp_plane<T, 256> : k_damp_plane<T, 512>;
 }
 
 template <typename T>
