@@ -197,7 +197,8 @@ int sparc_hip_sync(sparc_ctx* ctx);
 int sparc_hip_timing(sparc_ctx* ctx, int enable);
 int sparc_hip_kernel_time(sparc_ctx* ctx, int kind, long* count, double* total_ms);
 
-/* Tile (x, y, z-chunk) the stage kernel uses and its launch size. */
+/* Tile (x, y, z-chunk) the stage kernel of a run advanced alone uses and its
+ * launch size. */
 int sparc_hip_tile(sparc_ctx* ctx, int tile[3], long* nblocks);
 
 /* Tile autotuner (no counterpart in the reference; it serves the batched and
@@ -245,6 +246,10 @@ int sparc_hip_batch_advance(sparc_batch* b, int nsteps, const int* time0, const 
                             int flags);
 int sparc_hip_batch_filter(sparc_batch* b, const int* time);
 int sparc_hip_batch_info(sparc_batch* b, int* ngroups, long* nlaunch_blocks);
+/* Planes per z chunk a batch created now would give this run: the chunk it was
+ * set to, or, where that is automatic (tile chunk 0), the batch's own rule,
+ * which is not that of a run advanced alone (sparc_hip_tile). */
+int sparc_hip_batch_chunk(sparc_ctx* ctx, int* planes);
 int sparc_hip_batch_destroy(sparc_batch* b);
 /* Time per middle RK stage of the whole batch (reps launches of every
  * group), for tuning the tile shape of a group of runs; leaves every run's

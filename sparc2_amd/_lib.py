@@ -63,7 +63,7 @@ EXPORTS = [
     "sparc_hip_batch_info", "sparc_hip_batch_destroy", "sparc_hip_alfven_search",
     "sparc_hip_get_slab", "sparc_hip_autotune", "sparc_hip_set_tile", "sparc_hip_batch_time_stage",
     "sparc_hip_set_guard", "sparc_hip_guard", "sparc_hip_batch_filter", "sparc_hip_stream_bench",
-    "sparc_hip_deriv_noalloc", "sparc_hip_device_memory",
+    "sparc_hip_deriv_noalloc", "sparc_hip_device_memory", "sparc_hip_batch_chunk",
 ]
 
 _lib = None
@@ -103,6 +103,7 @@ def lib() -> C.CDLL:
     L.sparc_hip_timing.argtypes = [vp, i]
     L.sparc_hip_kernel_time.argtypes = [vp, i, C.POINTER(C.c_long), C.POINTER(C.c_double)]
     L.sparc_hip_tile.argtypes = [vp, C.c_int * 3, C.POINTER(C.c_long)]
+    L.sparc_hip_batch_chunk.argtypes = [vp, C.POINTER(C.c_int)]
     L.sparc_hip_batch_create.argtypes = [C.POINTER(vp), i, i, C.POINTER(vp)]
     L.sparc_hip_batch_advance.argtypes = [vp, i, C.POINTER(C.c_int), DP, i]
     L.sparc_hip_batch_filter.argtypes = [vp, C.POINTER(C.c_int)]

@@ -40,10 +40,10 @@ def _time_stage(h, reps: int) -> float:
     return ms.value
 
 
-# z-chunk depths the batch tuner tries, as multiples of each run's automatic
-# chunk: a persistent block pays a fixed cost per work item (its staging
-# plan, the argument switch, a barrier), which deeper chunks spread over more
-# planes.
+# z-chunk depths the batch tuner tries, as multiples of the chunk a batch gives
+# each run by itself (Solver.batch_chunk, not the chunk of a run advanced
+# alone): a persistent block pays a fixed cost per work item (its staging plan,
+# the argument switch, a barrier), which deeper chunks spread over more planes.
 KC_MULT = (1, 2, 4)
 
 
@@ -64,8 +64,8 @@ def tune_tiles(solvers: Sequence[Solver], reps: int = 3, by_variant: bool = Fals
     """Tile autotuning for a batch.  Runs that share a kernel variant share
     one launch, so the shape is chosen per variant group, by timing a middle
     RK stage of that group's batched launch for every shape that fits all of
-    its grids, each at the runs' automatic z chunks and at KC_MULT times
-    them (timing leaves the runs' states unchanged).  Returns
+    its grids, each at the z chunks a batch takes by itself and at KC_MULT
+    times them (timing leaves the runs' states unchanged).  Returns
     {variant: (tx, ty, chunk multiple)} and leaves each run on its group's
     best choice."""
     groups: Dict[tuple, List[Solver]] = {}
@@ -86,7 +86,7 @@ def tune_tiles(solvers: Sequence[Solver], reps: int = 3, by_variant: bool = Fals
             except SparcError:
                 pass                    # the shape does not fit a new grid: time again
             else:
-                auto = [s.tile()[0][2] for s in members]
+                auto = [s.batch_chunk() for s in members]
                 _apply(members, t, auto, mult)
                 chosen[key] = (t[0], t[1], mult)
                 continue
@@ -97,7 +97,7 @@ def tune_tiles(solvers: Sequence[Solver], reps: int = 3, by_variant: bool = Fals
                     s.set_tile((t[0], t[1], 0))
             except SparcError:
                 continue
-            auto = [s.tile()[0][2] for s in members]
+            auto = [s.batch_chunk() for s in members]
             for mult in KC_MULT:
                 if mult > 1 and all(k * mult > s.cfg.nz for s, k in zip(members, auto)):
                     break

@@ -1504,6 +1504,22 @@ static int batch_filter(sparc_batch* b, sparc_ctx* c, int time) {
 // register staging, 431 with this).
 static bool batch_dma(const sparc_ctx* c) { return c->dma && c->tx == 16 && c->ty == 16; }
 
+// Planes per z chunk of a run in a batch: its own where it was set, else a rule
+// of the batch's: the runs' items share the persistent blocks, so a run's own
+// rounds do not matter here: 4-plane chunks (MHD xy kernel), or about 512
+// blocks of at least 2 planes (quiet).
+static int batch_chunk(const sparc_ctx* c) {
+  if (!c->kc_auto) return c->kc;
+  const long tiles = (long)c->ntx * c->nty, want = c->zp ? 16384 : 512;
+  return (int)std::min<long>(c->nz, std::max<long>(c->zp ? 4 : 2, (c->nz * tiles + want - 1) / want));
+}
+
+int sparc_hip_batch_chunk(sparc_ctx* c, int* planes) {
+  if (!c || !planes) return fail(SPARC_E_INVALID, "null argument");
+  *planes = batch_chunk(c);
+  return SPARC_OK;
+}
+
 int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, sparc_batch** out) {
   if (!runs || nrun < 1 || !out) return fail(SPARC_E_INVALID, "batch needs at least one run");
   *out = nullptr;
@@ -1565,14 +1581,8 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     g.kc.assign(g.members.size(), 0);
     for (size_t q = 0; q < g.members.size(); ++q) {
       sparc_ctx* c = b->runs[g.members[q]];
-      const int tiles = c->ntx * c->nty;
-      // the runs' items share the persistent blocks, so a run's own rounds do
-      // not matter here: 4-plane chunks (MHD xy kernel), or about 512 blocks
-      // of at least 2 planes (quiet)
-      const int want = g.zp ? 16384 : 512;
-      g.kc[q] = !c->kc_auto ? c->kc
-                            : std::min(c->nz, (int)std::max<long>(g.zp ? 4 : 2, ((long)c->nz * tiles + want - 1) / want));
-      const int items = tiles * ((c->nz + g.kc[q] - 1) / g.kc[q]);
+      g.kc[q] = batch_chunk(c);
+      const int items = c->ntx * c->nty * ((c->nz + g.kc[q] - 1) / g.kc[q]);
       if ((rc = grow_partial(c, items))) return bail(rc);
       nblk_of[g.members[q]] = items;
       start[q + 1] = start[q] + items;

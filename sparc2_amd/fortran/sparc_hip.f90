@@ -58,6 +58,7 @@ module sparc_hip
        sparc_hip_autotune, sparc_hip_set_tile, sparc_hip_batch_time_stage, sparc_hip_set_damping, &
        sparc_hip_set_forcing, sparc_hip_set_guard, sparc_hip_guard, sparc_hip_batch_filter, &
        sparc_hip_stream_bench, sparc_hip_deriv_noalloc, sparc_hip_device_memory, &
+       sparc_hip_batch_chunk, &
        sparc_error_message
 
   interface
@@ -307,6 +308,12 @@ module sparc_hip
       type(c_ptr), value :: batch
       integer(c_int), intent(out) :: ngroups
       integer(c_long), intent(out) :: nlaunch_blocks
+    end function
+
+    integer(c_int) function sparc_hip_batch_chunk(ctx, planes) bind(C, name="sparc_hip_batch_chunk")
+      import :: c_int, c_ptr
+      type(c_ptr), value :: ctx
+      integer(c_int), intent(out) :: planes
     end function
 
     integer(c_int) function sparc_hip_batch_time_stage(batch, reps, ms_out) &

@@ -378,6 +378,12 @@ class Solver:
         t = (C.c_int * 3)(*[int(v) for v in tile])
         check(lib().sparc_hip_set_tile(self.h, t), "sparc_hip_set_tile")
 
+    def batch_chunk(self) -> int:
+        """Planes per z chunk a batch created now would give this run."""
+        k = C.c_int()
+        check(lib().sparc_hip_batch_chunk(self.h, C.byref(k)), "sparc_hip_batch_chunk")
+        return k.value
+
     def tile_key(self) -> tuple:
         """What the best tile depends on: grid, physics variant, precision,
         boundary kind, CPML widths and the points per lane (SPARC_LANE_POINTS
