@@ -160,6 +160,7 @@ struct sparc_ctx {
   int tx = 64, ty = 8, kc = 8, ntx = 1, nty = 1, nchunk = 1;
   int zn = 1;  // z-pass chunks
   bool kc_auto = true;       // kc follows auto_chunk
+  bool tile_auto = false;    // the shape follows choose_tile
   int ncu = 256;
   bool bg_set = false, state_set = false;
   // the uploaded rhoinv is bitwise 1/rho0 (initialize.f90:1012) at every point
@@ -385,54 +386,69 @@ static bool tile_fits(const sparc_ctx* c, int tx, int ty) {
 static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost);
 static void set_geometry(sparc_ctx* c, int tx, int ty, int kc);
 
+struct Shape {
+  int tx, ty;
+};
+static constexpr int kShapes = 4;
+
+// Grids whose rows are not whole 128-byte lines: a tile's row of 128 bytes
+// (16 lanes of 8) then touches two lines and one of 256 bytes three, so
+// the wider tile fetches a quarter less (MHD FP64 191x175x130, best chunk
+// of each shape: 16x16 588 us, 32x8 492, 32x16 481; 150x90x120 233 / - /
+// 201; quiet FP64 250x130x140 222 / 182 / 171).  Two-point FP32 MHD lanes
+// stay at 16x16 (150x90x120: 113 us, 32x16 129).
+static bool whole_lines(const sparc_ctx* c) { return (size_t)c->nx * c->esz % 128 == 0; }
+
+static const Shape quiet64[kShapes] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
+static const Shape quiet64m[kShapes] = {{32, 16}, {32, 8}, {16, 16}, {64, 4}};
+static const Shape quiet32[kShapes] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
+static const Shape* mhd_shapes(const sparc_ctx* c, bool lines) {
+  static const Shape mhd64[kShapes] = {{16, 16}, {32, 16}, {32, 8}, {64, 4}};
+  static const Shape mhd64m[kShapes] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
+  static const Shape mhd32[kShapes] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
+  // two points per lane (FP32, even nx): the MHD xy kernel at 16x16 lanes
+  static const Shape mhd32x2[kShapes] = {{16, 16}, {32, 8}, {32, 16}, {64, 4}};
+  return c->f32 ? (c->vw == 2 ? mhd32x2 : mhd32) : (lines ? mhd64 : mhd64m);
+}
+
+// A plane of more than 512 tiles of 32x8 takes 32x16 tiles, which re-read
+// fewer halo rows (512x512x300 FP64, one stage in 300-plane chunks: 32x8
+// 2.31 ms, 32x16 2.04 ms).
+static bool large_plane(const sparc_ctx* c) {
+  return (long)((c->nx + 32 * c->vw - 1) / (32 * c->vw)) * ((c->ny + 7) / 8) > 512;
+}
+
 static void choose_tile(sparc_ctx* c) {
   const sparc_cfg& q = c->cfg;
   int tx = q.tile[0], ty = q.tile[1];
   if (!(tx > 0 && ty > 0 && stage_tile_supported(tx, ty))) {
-    // Grids whose rows are not whole 128-byte lines: a tile's row of 128 bytes
-    // (16 lanes of 8) then touches two lines and one of 256 bytes three, so
-    // the wider tile fetches a quarter less (MHD FP64 191x175x130, best chunk
-    // of each shape: 16x16 588 us, 32x8 492, 32x16 481; 150x90x120 233 / - /
-    // 201; quiet FP64 250x130x140 222 / 182 / 171).  Two-point FP32 MHD lanes
-    // stay at 16x16 (150x90x120: 113 us, 32x16 129).
-    const bool lines = (size_t)c->nx * c->esz % 128 == 0;
-    static const int quiet64[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
-    static const int quiet64m[4][2] = {{32, 16}, {32, 8}, {16, 16}, {64, 4}};
-    static const int quiet32[4][2] = {{32, 8}, {16, 16}, {32, 16}, {64, 4}};
-    static const int mhd64[4][2] = {{16, 16}, {32, 16}, {32, 8}, {64, 4}};
-    static const int mhd64m[4][2] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
-    static const int mhd32[4][2] = {{32, 8}, {32, 16}, {16, 16}, {64, 4}};
-    // two points per lane (FP32, even nx): the MHD xy kernel at 16x16 lanes
-    static const int mhd32x2[4][2] = {{16, 16}, {32, 8}, {32, 16}, {64, 4}};
-    const int(*pref)[2] = c->mhd ? (c->f32 ? (c->vw == 2 ? mhd32x2 : mhd32) : (lines ? mhd64 : mhd64m))
-                                 : (c->f32 ? quiet32 : (lines ? quiet64 : quiet64m));
+    const bool lines = whole_lines(c);
+    const Shape* pref = c->mhd ? mhd_shapes(c, lines) : (c->f32 ? quiet32 : (lines ? quiet64 : quiet64m));
     tx = 32;
     ty = 8;
     double least = 1e300;
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < kShapes; ++n) {
+      const Shape& p = pref[n];
       // narrow grids: a 16-wide tile wastes less of each block
-      if (c->nx <= 16 && pref[n][0] * c->vw > 16) continue;
-      if (!tile_fits(c, pref[n][0], pref[n][1])) continue;
+      if (c->nx <= 16 && p.tx * c->vw > 16) continue;
+      if (!tile_fits(c, p.tx, p.ty)) continue;
       // the MHD shapes in order of preference; a quiet run takes the shape
       // whose launch is shortest (auto_chunk, with 15% for the second line of
       // 128-byte rows), the preferred of equal ones
       double cost = 0.0;
       if (!c->mhd) {
-        auto_chunk(c, pref[n][0], pref[n][1], &cost);
-        if (!lines) cost *= 1.0 + 0.15 * 128.0 / (double)(pref[n][0] * c->vw * c->esz);
+        auto_chunk(c, p.tx, p.ty, &cost);
+        if (!lines) cost *= 1.0 + 0.15 * 128.0 / (double)(p.tx * c->vw * c->esz);
       }
       if (cost < least) {
         least = cost;
-        tx = pref[n][0];
-        ty = pref[n][1];
+        tx = p.tx;
+        ty = p.ty;
       }
       if (c->mhd) break;
     }
-    // a plane of more than 512 tiles of 32x8 takes 32x16 tiles, which re-read
-    // fewer halo rows (512x512x300 FP64, one stage in 300-plane chunks: 32x8
-    // 2.31 ms, 32x16 2.04 ms)
-    const long t32x8 = (long)((c->nx + 32 * c->vw - 1) / (32 * c->vw)) * ((c->ny + 7) / 8);
-    if (!c->mhd && ty == 8 && t32x8 > 512 && tile_fits(c, 32, 16)) ty = 16;
+    if (!c->mhd && ty == 8 && large_plane(c) && tile_fits(c, 32, 16)) ty = 16;
+    c->tile_auto = true;
   }
   set_geometry(c, tx, ty, q.tile[2]);
 }
@@ -1288,6 +1304,7 @@ static int grow_partial(sparc_ctx* c, long nblk) {
 static int retile(sparc_ctx* c, int tx, int ty, int kc) {
   if (!tile_fits(c, tx, ty)) return fail(SPARC_E_INVALID, "tile shape unsupported or does not fit the grid");
   set_geometry(c, tx, ty, kc);
+  c->tile_auto = false;
   return grow_partial(c, (long)c->ntx * c->nty * c->nchunk);
 }
 
@@ -1389,6 +1406,7 @@ struct BatchGroup {
   bool mhd = false, bg3d = false, zp = false, dma = false;
   int vw = 1, tx = 0, ty = 0, nblk = 0, znblk = 0;
   std::vector<int> members;
+  std::vector<int> ntx, ntile; // tiles along x, and in a plane, per member
   std::vector<int> kc;         // z chunk depth per member in this batch
   std::vector<int> zn;         // z-pass chunks per member in this batch
   void* args[5] = {};         // StageArgs<T>[members] per stage (device)
@@ -1441,6 +1459,8 @@ static int batch_upload_args(sparc_batch* b) {
         sparc_ctx* c = b->runs[r];
         fill_common<T>(c, h[q]);
         set_stage<T>(c, h[q], s);
+        h[q].ntx = g.ntx[q];
+        h[q].nblk_xy = g.ntile[q];
         h[q].kc = g.kc[q];
         if (g.zp) h[q].zn = g.zn[q];
         h[q].amp_tab = c->cfg.pulse_dir ? (const T*)b->amp[r] : nullptr;
@@ -1499,24 +1519,77 @@ static int batch_filter(sparc_batch* b, sparc_ctx* c, int time) {
   return SPARC_OK;
 }
 
-// The batched MHD xy kernel stages with direct-to-LDS loads where a single
-// run's does (six 0.3 to 1.3 M point runs, z pass and stage: FP32 447 us with
-// register staging, 431 with this).
-static bool batch_dma(const sparc_ctx* c) { return c->dma && c->tx == 16 && c->ty == 16; }
+// The batched MHD xy kernel stages with direct-to-LDS loads where every run of
+// its launch can (six 0.3 to 1.3 M point runs, z pass and stage: FP32 447 us with
+// register staging, 431 with this); runs that cannot do not get a launch of
+// their own (96x96x120 and 90x96x120, FP32: 298 us in two launches, 219 in one
+// with register staging; 96x96x120 and 91x96x120 on 16x16 tiles, FP64: 455, 381).
+static bool can_dma(const sparc_ctx* c, Shape t) { return c->dma && t.tx == 16 && t.ty == 16; }
 
-// Planes per z chunk of a run in a batch: its own where it was set, else a rule
-// of the batch's: the runs' items share the persistent blocks, so a run's own
-// rounds do not matter here: 4-plane chunks (MHD xy kernel), or about 512
-// blocks of at least 2 planes (quiet).
-static int batch_chunk(const sparc_ctx* c) {
+static bool same_variant(const sparc_ctx* a, const sparc_ctx* b) {
+  return a->mhd == b->mhd && a->bg3d == b->bg3d && a->zp == b->zp && a->vw == b->vw;
+}
+
+// Tile shape of run c in a batch.  The launches of a batch follow one another,
+// each with a start and an end that leave part of the chip idle, so where the
+// automatic shapes of a variant's runs differ, they share one that fits them all:
+// MHD the first in the order of choose_tile, quiet the one that most of the
+// points have.  A stage, each run in its own shape against one for all: FP64 MHD
+// six runs of 0.4 to 1.6 M points 1044 us in three launches, 980 in one, two of
+// 1.1 M 424, 349; FP64 quiet six of 0.2 to 3.3 M 427, 344, two of 4.5 and 5.9 M
+// 469, 392; FP32 quiet two of 2 M 139, 103, five of 1 to 2 M 246, 195; 3-D
+// backgrounds FP64 511, 459, FP32 354, 283.  (Slower where one run has half of
+// the work: FP32 160x160x128 with five smaller ones 210, 240.)  A shape that was
+// set stays, and so does that of a run of 8 million points or more, to which a
+// launch of its own is nothing (384x384x160 with 64x64x128 and 160x160x128, FP32:
+// 972 us in one launch, 636 in two; 256x256x160 with 64x64x128 and 200x150x150,
+// FP64: 800, 633).
+static Shape batch_shape(const std::vector<sparc_ctx*>& runs, const sparc_ctx* c) {
+  const Shape own = {c->tx, c->ty};
+  auto shares = [&](const sparc_ctx* r) {
+    return same_variant(r, c) && r->tile_auto && r->N < 8'000'000;
+  };
+  if (!shares(c)) return own;
+  bool lines = true, differ = false;
+  for (const sparc_ctx* r : runs) {
+    if (!shares(r)) continue;
+    lines = lines && whole_lines(r);
+    differ = differ || r->tx != c->tx || r->ty != c->ty;
+  }
+  if (!differ) return own;
+  const Shape* pref = c->mhd ? mhd_shapes(c, lines) : quiet64;
+  Shape best = own;
+  long most = -1;
+  for (int n = 0; n < kShapes; ++n) {
+    const Shape t = pref[n];
+    long points = 0;
+    bool fits = true;
+    for (const sparc_ctx* r : runs) {
+      if (!shares(r)) continue;
+      fits = fits && tile_fits(r, t.tx, t.ty);
+      if (!r->mhd && r->tx == t.tx && r->ty == t.ty) points += r->N;
+    }
+    if (fits && points > most) {
+      best = t;
+      most = points;
+    }
+  }
+  return best;
+}
+
+// Planes per z chunk of a run of `tiles` tiles in a batch: its own where it was
+// set, else a rule of the batch's: the runs' items share the persistent blocks,
+// so a run's own rounds do not matter here: 4-plane chunks (MHD xy kernel), or
+// about 512 blocks of at least 2 planes (quiet).
+static int batch_chunk(const sparc_ctx* c, long tiles) {
   if (!c->kc_auto) return c->kc;
-  const long tiles = (long)c->ntx * c->nty, want = c->zp ? 16384 : 512;
+  const long want = c->zp ? 16384 : 512;
   return (int)std::min<long>(c->nz, std::max<long>(c->zp ? 4 : 2, (c->nz * tiles + want - 1) / want));
 }
 
 int sparc_hip_batch_chunk(sparc_ctx* c, int* planes) {
   if (!c || !planes) return fail(SPARC_E_INVALID, "null argument");
-  *planes = batch_chunk(c);
+  *planes = batch_chunk(c, (long)c->ntx * c->nty);
   return SPARC_OK;
 }
 
@@ -1555,11 +1628,10 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->dev);
   for (int r = 0; r < nrun; ++r) {
     sparc_ctx* c = b->runs[r];
+    const Shape t = batch_shape(b->runs, c);
     BatchGroup* g = nullptr;
     for (auto& h : b->groups)
-      if (h.mhd == c->mhd && h.bg3d == c->bg3d && h.zp == c->zp && h.vw == c->vw && h.tx == c->tx &&
-          h.ty == c->ty && h.dma == batch_dma(c))
-        g = &h;
+      if (same_variant(b->runs[h.members[0]], c) && h.tx == t.tx && h.ty == t.ty) g = &h;
     if (!g) {
       b->groups.emplace_back();
       g = &b->groups.back();
@@ -1567,11 +1639,14 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
       g->bg3d = c->bg3d;
       g->zp = c->zp;
       g->vw = c->vw;
-      g->tx = c->tx;
-      g->ty = c->ty;
-      g->dma = batch_dma(c);
+      g->tx = t.tx;
+      g->ty = t.ty;
+      g->dma = true;
     }
+    g->dma = g->dma && can_dma(c, t);
     g->members.push_back(r);
+    g->ntx.push_back((c->nx + t.tx * c->vw - 1) / (t.tx * c->vw));
+    g->ntile.push_back(g->ntx.back() * ((c->ny + t.ty - 1) / t.ty));
   }
   const size_t asz = b->f32 ? sizeof(StageArgs<float>) : sizeof(StageArgs<double>);
   std::vector<int> nblk_of(nrun, 0);  // diagnostic partials per run
@@ -1581,8 +1656,8 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     g.kc.assign(g.members.size(), 0);
     for (size_t q = 0; q < g.members.size(); ++q) {
       sparc_ctx* c = b->runs[g.members[q]];
-      g.kc[q] = batch_chunk(c);
-      const int items = c->ntx * c->nty * ((c->nz + g.kc[q] - 1) / g.kc[q]);
+      g.kc[q] = batch_chunk(c, g.ntile[q]);
+      const int items = g.ntile[q] * ((c->nz + g.kc[q] - 1) / g.kc[q]);
       if ((rc = grow_partial(c, items))) return bail(rc);
       nblk_of[g.members[q]] = items;
       start[q + 1] = start[q] + items;
