@@ -12,9 +12,9 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -167,11 +167,8 @@ struct sparc_ctx {
   bool rinv_rho0 = false;
   long steps_done = 0;
   double* op_buf = nullptr;  // 2*N doubles for the standalone operators
-  // read-out (download_all): pinned slots of pin_piece doubles and their events
-  double* pin = nullptr;
-  long pin_piece = 0;
-  int pin_slots = 0;
-  hipEvent_t pin_ev[2 * 8] = {};
+  bool reads = false;        // counted in its device's Reader
+  void* pin = nullptr;       // kGuardBytes of pinned memory, or null
   bool timing = false;
   std::vector<TimeRec> trecs;
   long tcount[5] = {0, 0, 0, 0, 0};
@@ -186,6 +183,7 @@ static bool stage_tile_supported(int tx, int ty) {
 // z-pass work items: blocks of 256 columns x z chunks
 static long zpass_items(int nx, int ny, int nchunk) { return ((long)nx * ny + 255) / 256 * nchunk; }
 
+static constexpr int kMaxDevices = 64;
 static constexpr size_t kGuardBytes = sizeof(double) * 4 + sizeof(int) * G_WORDS;
 
 static long round_up(long v, long m) { return (v + m - 1) / m * m; }
@@ -222,11 +220,15 @@ static int upload(sparc_ctx* c, void* dst, const double* src, long n) {
 // small pinned buffers, and every page of a fresh result array is touched for
 // the first time by that one thread -- and FP32 values were converted by it
 // as well (384x384x160, five fields: 91 ms FP64, 255 ms FP32).  Instead the pieces of
-// all arrays pass through the context's own pinned slots, two per worker
-// thread: a worker's next piece crosses the link while it copies the last one
-// out, and a kernel writes the slots, widening FP32 values on the way: 21 ms in
-// both (46 GB/s of the link's 57; copies by the DMA engine 24 ms in FP64 and
-// 1.0 against 0.85 ms for 64x64x128, by their start-up).
+// all arrays pass through pinned slots, two per worker thread: a worker's next
+// piece crosses the link while it copies the last one out, and a kernel writes
+// the slots, widening FP32 values on the way: 21 ms in both (46 GB/s of the
+// link's 57; copies by the DMA engine 24 ms in FP64 and 1.0 against 0.85 ms for
+// 64x64x128, by their start-up).
+//
+// The slots (32 MiB) belong to the device: its contexts take turns, since one
+// read-out fills the link.  The first read-out makes them (0.6 ms) and the last
+// context gives them back.  Without them results are copied plainly.
 // ---------------------------------------------------------------------------
 struct Segment {
   double* dst;
@@ -236,49 +238,111 @@ struct Segment {
   bool f32;
 };
 
-static constexpr int kMaxReaders = 8;
+static constexpr int kMaxReaders = 8, kMaxSegments = 8 + 6;
+// an FP64 result up to this size is copied plainly: 18 KB 11 us, through the
+// slots 15; 512 KB 34 and 35; 1152 KB 97 and 72
+static constexpr size_t kPlainBytes = 512u << 10;
+static constexpr size_t kSlotBytes = 2u << 20, kSlot = kSlotBytes / sizeof(double);
 
-// pinned slots for results of `bytes`: pieces of 2 MiB, fewer threads and
-// smaller pieces for small results (a thread costs about 30 us to start)
-static void reader_shape(size_t bytes, int* workers, long* piece) {
-  *workers = (int)std::min<size_t>(kMaxReaders, std::max<size_t>(1, bytes >> 22));
-  const size_t p = std::min<size_t>(2u << 20, std::max<size_t>(256u << 10, bytes / (4 * *workers)));
-  *piece = (long)(p / sizeof(double) / 1024 * 1024);
+namespace {
+struct Reader {
+  std::mutex mu;
+  int contexts = 0;
+  double* pin = nullptr;  // 2 * kMaxReaders slots
+  hipEvent_t ev[2 * kMaxReaders] = {};
+};
+Reader g_reader[kMaxDevices];
+}  // namespace
+
+static void reader_free(Reader& r) {
+  if (r.pin) (void)hipHostFree(r.pin);
+  r.pin = nullptr;
+  for (auto& e : r.ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
+  }
 }
 
-static int reader_create(sparc_ctx* c) {
-  int workers;
-  long piece;
-  reader_shape(sizeof(double) * (size_t)c->nv * c->N, &workers, &piece);
-  c->pin_slots = 2 * workers;
-  c->pin_piece = piece;
-  if (hipHostMalloc((void**)&c->pin, sizeof(double) * piece * c->pin_slots, hipHostMallocDefault) != hipSuccess) {
-    c->pin = nullptr;
-    return fail(SPARC_E_NOMEM, "pinned read-out memory");
-  }
-  for (int q = 0; q < c->pin_slots; ++q)
-    if (hipEventCreateWithFlags(&c->pin_ev[q], hipEventDisableTiming) != hipSuccess) {
-      c->pin_ev[q] = nullptr;
-      return fail(SPARC_E_HIP, "read-out event");
+// With the lock held: whether the slots are there.
+static bool reader_slots(Reader& r) {
+  if (r.pin) return true;
+  bool ok = hipHostMalloc((void**)&r.pin, kSlotBytes * 2 * kMaxReaders, hipHostMallocDefault) == hipSuccess;
+  if (!ok) r.pin = nullptr;
+  for (auto& e : r.ev)
+    if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      e = nullptr;
+      ok = false;
     }
+  if (!ok) {
+    reader_free(r);
+    (void)hipGetLastError();
+  }
+  return ok;
+}
+
+static void reader_join(sparc_ctx* c) {
+  std::lock_guard<std::mutex> lock(g_reader[c->dev].mu);
+  g_reader[c->dev].contexts++;
+  c->reads = true;
+}
+
+static void reader_leave(sparc_ctx* c) {
+  if (!c->reads) return;
+  Reader& r = g_reader[c->dev];
+  std::lock_guard<std::mutex> lock(r.mu);
+  c->reads = false;
+  if (--r.contexts == 0) reader_free(r);
+}
+
+// One array in plain copies; an FP32 one in pieces, widened here.
+static int download_plain(sparc_ctx* c, const Segment& g) {
+  if (!g.f32) {
+    HIPCHK(hipMemcpyAsync(g.dst, g.src, sizeof(double) * g.n, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    return SPARC_OK;
+  }
+  constexpr long kPiece = 16384;
+  float v[kPiece];
+  uint16_t w[kPiece];
+  for (long at = 0; at < g.n; at += kPiece) {
+    const long n = std::min(kPiece, g.n - at);
+    HIPCHK(hipMemcpyAsync(v, (const float*)g.src + at, sizeof(float) * n, hipMemcpyDeviceToHost, c->st));
+    if (g.comp)
+      HIPCHK(hipMemcpyAsync(w, (const uint16_t*)g.comp + at, sizeof(uint16_t) * n, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    for (long q = 0; q < n; ++q) g.dst[at + q] = g.comp ? (double)v[q] - (double)bf2f(w[q]) : (double)v[q];
+  }
+  return SPARC_OK;
+}
+
+// A few bytes through the context's own pinned ones: 14 us, from pageable
+// memory 22.
+static int download_small(sparc_ctx* c, void* dst, const void* src, size_t n) {
+  void* const h = c->pin ? c->pin : dst;
+  HIPCHK(hipMemcpyAsync(h, src, n, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  if (h != dst) memcpy(dst, h, n);
   return SPARC_OK;
 }
 
 static int download_all(sparc_ctx* c, const Segment* seg, int nseg) {
-  struct Piece {
-    const Segment* s;
-    long at, n;
-  };
-  std::vector<Piece> pieces;
   size_t bytes = 0;
   for (int q = 0; q < nseg; ++q) bytes += sizeof(double) * (size_t)seg[q].n;
-  int workers;
-  long piece;
-  reader_shape(bytes, &workers, &piece);
-  workers = std::min(workers, c->pin_slots / 2);
-  piece = std::min(piece, c->pin_piece);
-  for (int q = 0; q < nseg; ++q)
-    for (long at = 0; at < seg[q].n; at += piece) pieces.push_back({&seg[q], at, std::min(piece, seg[q].n - at)});
+  if (nseg == 1 && !seg[0].f32 && bytes <= kPlainBytes) return download_plain(c, seg[0]);
+  Reader& r = g_reader[c->dev];
+  std::lock_guard<std::mutex> lock(r.mu);
+  if (!reader_slots(r)) {
+    for (int q = 0; q < nseg; ++q)
+      if (int rc = download_plain(c, seg[q])) return rc;
+    return SPARC_OK;
+  }
+  // pieces of 2 MiB; fewer threads and smaller pieces for small results (a
+  // thread costs about 30 us to start)
+  const int workers = (int)std::min<size_t>(kMaxReaders, std::max<size_t>(1, bytes >> 22));
+  const long piece =
+      (long)(std::min(kSlotBytes, std::max<size_t>(256u << 10, bytes / (4 * workers))) / sizeof(double) / 1024 * 1024);
+  size_t first[kMaxSegments + 1] = {};  // each array's first piece
+  for (int q = 0; q < nseg; ++q) first[q + 1] = first[q] + (size_t)((seg[q].n + piece - 1) / piece);
   std::atomic<size_t> next{0};
   std::atomic<int> error{(int)hipSuccess};
   // one worker: its two slots in turn
@@ -287,41 +351,41 @@ static int download_all(sparc_ctx* c, const Segment* seg, int nseg) {
       error = (int)hipErrorInvalidDevice;
       return;
     }
-    Piece held{nullptr, 0, 0};
-    int slot = 0, held_slot = 0;
-    for (;;) {
+    double* held = nullptr;  // where the other slot's piece goes
+    long held_n = 0;
+    for (int slot = 2 * w, s = 0;; slot ^= 1) {
       const size_t i = next.fetch_add(1);
       hipError_t e = hipSuccess;
-      if (i < pieces.size()) {
-        const Piece& p = pieces[i];
-        double* const pin = c->pin + (size_t)(2 * w + slot) * c->pin_piece;
-        if (p.s->f32)
-          e = launch_widen((const float*)p.s->src + p.at, p.s->comp ? (const uint16_t*)p.s->comp + p.at : nullptr,
-                           pin, p.n, c->st);
+      double* dst = nullptr;
+      long n = 0;
+      if (i < first[nseg]) {
+        while (i >= first[s + 1]) ++s;
+        const Segment& g = seg[s];
+        const long at = (long)(i - first[s]) * piece;
+        n = std::min(piece, g.n - at);
+        dst = g.dst + at;
+        double* const pin = r.pin + slot * kSlot;
+        if (g.f32)
+          e = launch_widen((const float*)g.src + at, g.comp ? (const uint16_t*)g.comp + at : nullptr, pin, n, c->st);
         else
-          e = launch_copy((const double*)p.s->src + p.at, pin, p.n, false, c->st, nullptr);
-        if (e == hipSuccess) e = hipEventRecord(c->pin_ev[2 * w + slot], c->st);
+          e = launch_copy((const double*)g.src + at, pin, n, false, c->st, nullptr);
+        if (e == hipSuccess) e = hipEventRecord(r.ev[slot], c->st);
       }
-      if (e == hipSuccess && held.s) {
-        e = hipEventSynchronize(c->pin_ev[2 * w + held_slot]);
-        if (e == hipSuccess)
-          memcpy(held.s->dst + held.at, c->pin + (size_t)(2 * w + held_slot) * c->pin_piece, sizeof(double) * held.n);
+      if (e == hipSuccess && held) {
+        e = hipEventSynchronize(r.ev[slot ^ 1]);
+        if (e == hipSuccess) memcpy(held, r.pin + (slot ^ 1) * kSlot, sizeof(double) * held_n);
       }
-      if (e != hipSuccess) {
-        error = (int)e;
-        return;
-      }
-      if (i >= pieces.size()) return;
-      held = pieces[i];
-      held_slot = slot;
-      slot ^= 1;
+      if (e != hipSuccess) error = (int)e;
+      if (e != hipSuccess || !dst) return;
+      held = dst;
+      held_n = n;
     }
   };
   std::thread pool[kMaxReaders];
   int started = 1;
   try {
     for (; started < workers; ++started) pool[started] = std::thread(work, started);
-  } catch (const std::system_error&) {  // fewer threads: the others take their pieces
+  } catch (const std::exception&) {  // fewer threads: the others take their pieces
   }
   work(0);
   for (int w = 1; w < started; ++w) pool[w].join();
@@ -351,9 +415,8 @@ static void free_all(sparc_ctx* c) {
   F(c->diag);
   F(c->gdiag);  // and the guard record in it
   F(c->op_buf);
+  reader_leave(c);
   if (c->pin) (void)hipHostFree(c->pin);
-  for (auto& e : c->pin_ev)
-    if (e) (void)hipEventDestroy(e);
   F(c->fmap);
   F(c->sdep);
   damp_destroy(c->damp);
@@ -567,7 +630,6 @@ static constexpr long kNoAllocMaxPoints = 1L << 22;  // 4,194,304 grid points
 static __device__ __align__(256) double scratch[2 * kNoAllocMaxPoints];
 
 namespace {
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 }  // namespace
@@ -657,6 +719,11 @@ int sparc_hip_create(const sparc_cfg* cfg, sparc_ctx** out) {
     return code;
   };
   if ((rc = scratch_setup(c->dev))) return bail(rc);
+  reader_join(c);
+  if (hipHostMalloc(&c->pin, kGuardBytes, hipHostMallocDefault) != hipSuccess) {
+    c->pin = nullptr;
+    (void)hipGetLastError();
+  }
   if (hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking) != hipSuccess)
     return bail(fail(SPARC_E_HIP, "hipStreamCreate failed"));
 
@@ -724,7 +791,6 @@ int sparc_hip_create(const sparc_cfg* cfg, sparc_ctx** out) {
     if (hipMemcpy(c->stretch_lo, lo.data(), sizeof(float) * q.nz, hipMemcpyHostToDevice) != hipSuccess)
       return bail(fail(SPARC_E_HIP, "stretch upload failed"));
   }
-  if ((rc = reader_create(c))) return bail(rc);
   if (hipMemcpy(c->stretch_d, q.stretch, sizeof(double) * q.nz, hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(SPARC_E_HIP, "stretch upload failed"));
   if (hipStreamSynchronize(c->st) != hipSuccess) return bail(fail(SPARC_E_HIP, "sync failed"));
@@ -1125,9 +1191,7 @@ int sparc_hip_diag(sparc_ctx* c, double out[3]) {
   if (c->steps_done == 0) return fail(SPARC_E_STATE, "no step taken yet");
   HIPCHK(hipSetDevice(c->dev));
   double h[3];
-  HIPCHK(hipMemcpyAsync(c->pin, c->diag, sizeof h, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
-  memcpy(h, c->pin, sizeof h);
+  if (int rc = download_small(c, h, c->diag, sizeof h)) return rc;
   const double nrm = std::pow(h[0] / ((double)c->nx * (double)c->ny * (double)c->nz), 0.5);
   out[0] = nrm * (c->dimc * c->dimc) * c->dimrho;
   out[1] = h[1];
@@ -1154,12 +1218,14 @@ int sparc_hip_guard(sparc_ctx* c, int* tripped, long* at_step, long* steps, doub
   if (!c) return fail(SPARC_E_INVALID, "null context");
   HIPCHK(hipSetDevice(c->dev));
   // both in one copy: the record follows the failing step's values
-  HIPCHK(hipMemcpyAsync(c->pin, c->gdiag, kGuardBytes, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipStreamSynchronize(c->st));
-  int g[G_WORDS];
-  double d[4];
-  memcpy(d, c->pin, sizeof d);
-  memcpy(g, c->pin + 4, sizeof g);
+  struct {
+    double d[4];
+    int g[G_WORDS];
+  } h;
+  static_assert(sizeof h == kGuardBytes, "the layout of gdiag");
+  if (int rc = download_small(c, &h, c->gdiag, sizeof h)) return rc;
+  const double* const d = h.d;
+  const int* const g = h.g;
   if (tripped) *tripped = g[G_TRIPPED];
   if (at_step) *at_step = g[G_TRIPPED] ? g[G_AT] : 0;
   if (steps) *steps = g[G_COUNT];
