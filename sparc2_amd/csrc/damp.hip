@@ -373,7 +373,7 @@ struct DampPlan {
   hipfftHandle fwd = 0, inv = 0;
   bool f32 = false;
   int nx = 0, ny = 0, nz = 0;
-  int nf = 1;             // fields per transform: 3, or 1 where the slabs are padded
+  int nf = 1;             // fields per library transform: 3 or 1
   long fs = 0;
   void* spec = nullptr;   // half spectra of nf fields, (nx/2+1)*ny*nz complex each
   void* rates = nullptr;  // (nx/2+1)*ny, element type
@@ -393,13 +393,19 @@ __global__ __launch_bounds__(256) void k_damp_mul(C* __restrict__ w, const T* __
   w[i] = v;
 }
 
-void damp_destroy(DampPlan* d) {
-  if (!d) return;
+static void library_free(DampPlan* d) {
   if (d->fwd) (void)hipfftDestroy(d->fwd);
   if (d->inv) (void)hipfftDestroy(d->inv);
+  if (d->spec) (void)hipFree(d->spec);
+  d->fwd = d->inv = 0;
+  d->spec = nullptr;
+}
+
+void damp_destroy(DampPlan* d) {
+  if (!d) return;
+  library_free(d);
   if (d->roots) (void)hipFree(d->roots);
   if (d->places) (void)hipFree(d->places);
-  if (d->spec) (void)hipFree(d->spec);
   if (d->rates) (void)hipFree(d->rates);
   if (d->term) (void)hipFree(d->term);
   delete d;
@@ -496,6 +502,27 @@ static bool plane_tables(DampPlan* d, const double* rates) {
                              (int)kLdsBytes) == hipSuccess;
 }
 
+// The library's plans and the half spectra for nf fields at a time.
+static bool library_plans(DampPlan* d, int nf, hipStream_t st) {
+  // n, embeddings in C order (slowest first): a plane is ny rows of nx reals
+  // or of nx/2+1 complex values; batch = the nz planes of each field
+  const int nx = d->nx, ny = d->ny, mx = nx / 2 + 1, m = mx * ny;
+  int n[2] = {ny, nx}, real_embed[2] = {ny, nx}, cplx_embed[2] = {ny, mx};
+  const size_t esz = d->f32 ? sizeof(float) : sizeof(double);
+  d->nf = nf;
+  bool ok = hipMalloc(&d->spec, 2 * esz * m * d->nz * nf) == hipSuccess;
+  ok = ok && hipfftPlanMany(&d->fwd, 2, n, real_embed, 1, nx * ny, cplx_embed, 1, m, d->f32 ? HIPFFT_R2C : HIPFFT_D2Z,
+                            d->nz * nf) == HIPFFT_SUCCESS;
+  ok = ok && hipfftPlanMany(&d->inv, 2, n, cplx_embed, 1, m, real_embed, 1, nx * ny, d->f32 ? HIPFFT_C2R : HIPFFT_Z2D,
+                            d->nz * nf) == HIPFFT_SUCCESS;
+  ok = ok && hipfftSetStream(d->fwd, st) == HIPFFT_SUCCESS && hipfftSetStream(d->inv, st) == HIPFFT_SUCCESS;
+  if (!ok) {
+    library_free(d);
+    (void)hipGetLastError();
+  }
+  return ok;
+}
+
 // rates: (nx/2+1, ny) Fortran order = C (ny, nx/2+1), FP64 from the host.
 // Returns nullptr on failure (and frees what it made).
 DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* rates, hipStream_t st) {
@@ -505,7 +532,6 @@ DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* r
   d->ny = ny;
   d->nz = nz;
   d->fs = fs;
-  d->nf = fs == (long)nx * ny * nz ? 3 : 1;
   const int mx = nx / 2 + 1;
   const long m = (long)mx * ny;
   const size_t esz = f32 ? sizeof(float) : sizeof(double);
@@ -517,9 +543,7 @@ DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* r
     damp_destroy(d);
     return nullptr;
   }
-  bool ok = hipMalloc(&d->spec, 2 * esz * m * nz * d->nf) == hipSuccess &&
-            hipMalloc(&d->rates, esz * m) == hipSuccess &&
-            hipMalloc(&d->term, esz * 3 * fs) == hipSuccess;
+  bool ok = hipMalloc(&d->rates, esz * m) == hipSuccess && hipMalloc(&d->term, esz * 3 * fs) == hipSuccess;
   if (ok) {
     if (f32) {
       std::vector<float> h(rates, rates + m);
@@ -528,14 +552,11 @@ DampPlan* damp_create(int nx, int ny, int nz, long fs, bool f32, const double* r
       ok = hipMemcpy(d->rates, rates, esz * m, hipMemcpyHostToDevice) == hipSuccess;
     }
   }
-  // n, embeddings in C order (slowest first): a plane is ny rows of nx reals
-  // or of nx/2+1 complex values; batch = the nz planes of each field
-  int n[2] = {ny, nx}, real_embed[2] = {ny, nx}, cplx_embed[2] = {ny, mx};
-  ok = ok && hipfftPlanMany(&d->fwd, 2, n, real_embed, 1, nx * ny, cplx_embed, 1, (int)m,
-                            f32 ? HIPFFT_R2C : HIPFFT_D2Z, nz * d->nf) == HIPFFT_SUCCESS;
-  ok = ok && hipfftPlanMany(&d->inv, 2, n, cplx_embed, 1, (int)m, real_embed, 1, nx * ny,
-                            f32 ? HIPFFT_C2R : HIPFFT_Z2D, nz * d->nf) == HIPFFT_SUCCESS;
-  ok = ok && hipfftSetStream(d->fwd, st) == HIPFFT_SUCCESS && hipfftSetStream(d->inv, st) == HIPFFT_SUCCESS;
+  // Three fields in one transform where the slabs are unpadded, within 65535 rows
+  // of a launch and 2^31 values of a transform; one by one beyond, and where
+  // there is no memory for three fields' spectra.
+  const bool small = 3L * nz <= 65535 && 3L * fs < (1L << 31);
+  ok = ok && ((fs == (long)nx * ny * nz && small && library_plans(d, 3, st)) || library_plans(d, 1, st));
   if (!ok) {
     damp_destroy(d);
     return nullptr;
