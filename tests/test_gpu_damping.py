@@ -1,6 +1,7 @@
-"""FFT damping on the GPU (hipFFT r2c/c2r per z plane, the rates multiply,
-the term subtracted after the boundary zeroing) against the oracle's direct
-DFT sums, through the C ABI.  Bar: FP64 relative L2 1e-11 per field after N
+"""FFT damping on the GPU (each z plane's transforms and the rates multiply in
+one block, or by hipFFT where a plane does not suit that; the term subtracted
+after the boundary zeroing) against the oracle's direct DFT sums, through the C
+ABI.  Bar: FP64 relative L2 1e-11 per field after N
 driver steps; FP32 (two-point lanes, Kahan update) within 1e-5 of FP64."""
 import numpy as np
 import pytest

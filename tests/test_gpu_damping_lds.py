@@ -1,7 +1,7 @@
 """FFT damping of planes that a block transforms in LDS, against the oracle's
-direct DFT sums: every radix at the ends and inside of a transform, odd sides,
-one to three passes, columns left over from whole waves, padded and unpadded
-slabs, and the three block sizes.  Bars as in test_gpu_damping.py: FP64
+direct DFT sums: radices at the ends and inside of a transform (radix 2 is in
+test_gpu_damping_paths.py), odd sides, one to three passes, padded and unpadded
+slabs, and both block sizes.  Bars as in test_gpu_damping.py: FP64
 relative L2 1e-11 per field after the steps, FP32 within 1e-5 of FP64."""
 import numpy as np
 import pytest

@@ -1,6 +1,6 @@
-"""FFT damping where the field slabs are padded (each field transformed by
-itself) and where they are not (the three fields in one transform), against the
-oracle's direct DFT sums; odd and even plane sizes.  Bar as in
+"""FFT damping where the field slabs are padded and where they are not (where the
+library transforms the planes: each field by itself, or three in one), against
+the oracle's direct DFT sums; odd and even plane sizes.  Bar as in
 test_gpu_damping.py: FP64 relative L2 1e-11 per field after the steps."""
 import pytest
 
