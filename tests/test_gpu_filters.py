@@ -2,9 +2,10 @@
 
 The y and x passes run as one kernel: a wave owns 64 consecutive x points
 and writes the inner 52 (g = 5) or 56 (g = 3) of them, reading the x stencil
-from the neighbouring lanes; it marches up chunks of 64 rows.  The grids
+from the neighbouring lanes; it marches up chunks of rows, 16 of them on
+grids this small (longer chunks: test_gpu_filter_rings.py).  The grids
 here put nx below, at and just above one wave's output width and ny across
-two row chunks, periodic and not, with both filter widths, so every lane
+row chunks, periodic and not, with both filter widths, so every lane
 mask, wrap and chunk seam is exercised (non-periodic grids keep the stage
 kernels' rule of at least 6 cells in a boundary tile).  FP64 must equal the
 oracle to 1e-13 (the same arithmetic in the same order); the FP32 form
