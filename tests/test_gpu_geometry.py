@@ -1,7 +1,7 @@
 """The automatic launch geometry (tile shape, z chunk, z-pass chunk) against an
 explicit one: a stage computes every point by the same arithmetic whatever the
-split, so the states are equal bitwise.  Grids at the edges of the rule: one
-round of resident blocks, a few, ragged last chunks, the smallest axes."""
+split, so the states are equal bitwise.  Grids of one round of resident blocks,
+the smallest axes among them (several rounds: test_gpu_geometry_rounds.py)."""
 import numpy as np
 import pytest
 
