@@ -336,16 +336,6 @@ template <typename T> struct RowSum {
     else return p + s;
   }
 };
-struct RowSumF2 {
-  RowSum<float> a, b;
-  __device__ __forceinline__ void add(F2 v, int r, int m) {
-    a.add(v.x, r, m);
-    b.add(v.y, r, m);
-  }
-  __device__ __forceinline__ F2 sum() const { return F2(a.sum(), b.sum()); }
-};
-template <typename V> struct RowSumOf { using type = RowSum<V>; };
-template <> struct RowSumOf<F2> { using type = RowSumF2; };
 
 // The row tables copied into LDS, for the stage kernels: there the row of a
 // one-sided closure differs between the lanes of a wave, so reading the
@@ -368,6 +358,7 @@ template <typename T> struct RowTab {
     }
   }
 };
+
 // point c of a lane value
 template <typename T> __device__ __forceinline__ T lane_pt(T v, int) { return v; }
 __device__ __forceinline__ float lane_pt(F2 v, int c) { return c ? v.y : v.x; }
