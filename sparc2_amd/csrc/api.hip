@@ -193,6 +193,7 @@ static int dalloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();  // the next launch is not to report it
     return fail(SPARC_E_NOMEM, std::string("hipMalloc(") + std::to_string(bytes) + "): " +
                                    hipGetErrorString(e));
   }
@@ -1354,14 +1355,15 @@ int sparc_hip_kernel_time(sparc_ctx* c, int kind, long* count, double* total_ms)
   return SPARC_OK;
 }
 
-// Room for the diagnostic partials of nblk blocks.
+// Room for the diagnostic partials of nblk blocks; where there is no memory for
+// it the old buffer stays, and with it the run.
 static int grow_partial(sparc_ctx* c, long nblk) {
   if (nblk <= c->partial_cap) return SPARC_OK;
-  if (c->partial) (void)hipFree(c->partial);
-  c->partial = nullptr;
-  c->partial_cap = 0;
-  int rc = dalloc((void**)&c->partial, sizeof(double) * 3 * nblk);
+  double* p = nullptr;
+  int rc = dalloc((void**)&p, sizeof(double) * 3 * nblk);
   if (rc) return rc;
+  if (c->partial) (void)hipFree(c->partial);
+  c->partial = p;
   c->partial_cap = nblk;
   return SPARC_OK;
 }
@@ -1369,9 +1371,15 @@ static int grow_partial(sparc_ctx* c, long nblk) {
 // Re-tile a context between steps (the partial-sum buffer grows if needed).
 static int retile(sparc_ctx* c, int tx, int ty, int kc) {
   if (!tile_fits(c, tx, ty)) return fail(SPARC_E_INVALID, "tile shape unsupported or does not fit the grid");
+  const int old[3] = {c->tx, c->ty, c->kc_auto ? 0 : c->kc};
   set_geometry(c, tx, ty, kc);
+  const int rc = grow_partial(c, (long)c->ntx * c->nty * c->nchunk);
+  if (rc) {
+    set_geometry(c, old[0], old[1], old[2]);
+    return rc;
+  }
   c->tile_auto = false;
-  return grow_partial(c, (long)c->ntx * c->nty * c->nchunk);
+  return SPARC_OK;
 }
 
 int sparc_hip_set_tile(sparc_ctx* c, const int tile[3]) {
