@@ -1499,6 +1499,7 @@ struct sparc_batch {
   // work counters of the persistent launches (8 per-XCD item counters and a
   // count of the blocks that left; each launch leaves them zero)
   int* work = nullptr;
+  std::vector<int> nblk;   // diagnostic partials per run
   std::vector<void*> amp;  // per run, amp_cap entries (device)
   int amp_cap = 0;
   void* jobs = nullptr;    // DiagJob[nrun] (device)
@@ -1543,6 +1544,18 @@ static int batch_upload_args(sparc_batch* b) {
       HIPCHK(hipMemcpy(g.args[s - 1], h.data(), sizeof(StageArgs<T>) * h.size(), hipMemcpyHostToDevice));
     }
   }
+  // anew for each call, as the stage arguments are: set_tile or another batch
+  // may have given a run a longer buffer of partials
+  std::vector<DiagJob> jobs(b->runs.size());
+  for (size_t r = 0; r < jobs.size(); ++r) {
+    sparc_ctx* c = b->runs[r];
+    jobs[r].partial = c->partial;
+    jobs[r].out = c->diag;
+    jobs[r].nblk = b->nblk[r];
+    jobs[r].pad_ = 0;
+    jobs[r].g = guard_args(c);
+  }
+  HIPCHK(hipMemcpy(b->jobs, jobs.data(), sizeof(DiagJob) * jobs.size(), hipMemcpyHostToDevice));
   return SPARC_OK;
 }
 
@@ -1723,7 +1736,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     g->ntile.push_back(g->ntx.back() * ((c->ny + t.ty - 1) / t.ty));
   }
   const size_t asz = b->f32 ? sizeof(StageArgs<float>) : sizeof(StageArgs<double>);
-  std::vector<int> nblk_of(nrun, 0);  // diagnostic partials per run
+  b->nblk.assign(nrun, 0);
   int rc;
   for (auto& g : b->groups) {
     std::vector<int> start(g.members.size() + 1, 0);
@@ -1733,7 +1746,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
       g.kc[q] = batch_chunk(c, g.ntile[q]);
       const int items = g.ntile[q] * ((c->nz + g.kc[q] - 1) / g.kc[q]);
       if ((rc = grow_partial(c, items))) return bail(rc);
-      nblk_of[g.members[q]] = items;
+      b->nblk[g.members[q]] = items;
       start[q + 1] = start[q] + items;
     }
     for (int s = 0; s < 5; ++s)
@@ -1771,18 +1784,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
   if ((rc = dalloc((void**)&b->work, 16 * sizeof(int)))) return bail(rc);
   if (launch_zero(b->work, 16, true, b->st) != hipSuccess || hipStreamSynchronize(b->st) != hipSuccess)
     return bail(fail(SPARC_E_HIP, "work counter clear failed"));
-  std::vector<DiagJob> jobs(nrun);
-  for (int r = 0; r < nrun; ++r) {
-    sparc_ctx* c = b->runs[r];
-    jobs[r].partial = c->partial;
-    jobs[r].out = c->diag;
-    jobs[r].nblk = nblk_of[r];
-    jobs[r].pad_ = 0;
-    jobs[r].g = guard_args(c);
-  }
   if ((rc = dalloc(&b->jobs, sizeof(DiagJob) * nrun))) return bail(rc);
-  if (hipMemcpy(b->jobs, jobs.data(), sizeof(DiagJob) * nrun, hipMemcpyHostToDevice) != hipSuccess)
-    return bail(fail(SPARC_E_HIP, "diag job upload failed"));
   b->amp.assign(nrun, nullptr);
   *out = b;
   return SPARC_OK;
