@@ -475,6 +475,9 @@ static const Shape* mhd_shapes(const sparc_ctx* c, bool lines) {
   return c->f32 ? (c->vw == 2 ? mhd32x2 : mhd32) : (lines ? mhd64 : mhd64m);
 }
 
+// More state than the caches hold: the stage kernels are bound by memory there.
+static bool large_run(const sparc_ctx* c) { return c->N > 2'000'000; }
+
 // A plane of more than 512 tiles of 32x8 takes 32x16 tiles, which re-read
 // fewer halo rows (512x512x300 FP64, one stage in 300-plane chunks: 32x8
 // 2.31 ms, 32x16 2.04 ms).
@@ -497,12 +500,16 @@ static void choose_tile(sparc_ctx* c) {
       if (c->nx <= 16 && p.tx * c->vw > 16) continue;
       if (!tile_fits(c, p.tx, p.ty)) continue;
       // the MHD shapes in order of preference; a quiet run takes the shape
-      // whose launch is shortest (auto_chunk, with 15% for the second line of
-      // 128-byte rows), the preferred of equal ones
+      // whose launch is shortest (auto_chunk, with 20 %, large runs 30 %, for the
+      // second line of 128-byte rows), the preferred of equal ones.  Over 262
+      // runs of 0.2 to 9 M points this is within 1.5 % of the best shape on
+      // average; with 15 % for all and without regard to the waves of a round
+      // it was 2.7 %, and 79x134x136 FP32 took 297 us a step in 16x16 tiles
+      // against 229 in 32x8, 89x267x239 810 against 673 in 32x16.
       double cost = 0.0;
       if (!c->mhd) {
         auto_chunk(c, p.tx, p.ty, &cost);
-        if (!lines) cost *= 1.0 + 0.15 * 128.0 / (double)(p.tx * c->vw * c->esz);
+        if (!lines) cost *= 1.0 + (large_run(c) ? 0.3 : 0.2) * 128.0 / (double)(p.tx * c->vw * c->esz);
       }
       if (cost < least) {
         least = cost;
@@ -544,7 +551,11 @@ static int balanced_chunk(long tiles, int nz, long places, double c0, int kmax, 
 }
 
 // Automatic z chunk of the stage kernel on tx x ty tiles; cost: see
-// balanced_chunk (comparable between tile shapes of a variant).
+// balanced_chunk, and comparable between tile shapes of a variant: a round of
+// more resident lanes takes longer, in proportion where memory bounds it and by
+// about the root on small grids, whose waves wait for the caches (FP32 with one
+// point a lane: 768 blocks of 256 lanes are resident, or 256 of 512, whose round
+// takes 0.63 of the time on large grids and 0.83 on small ones).
 //  quiet: the window re-reads 10 planes of two fields per chunk, and a start
 //    takes as long as 4 planes (fitted over 48x48x96 .. 512x512x300);
 //  quiet with x and y CPML: the tiles at the sides take longer than the inner
@@ -566,7 +577,9 @@ static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost) {
     const bool lines = (size_t)c->nx * c->esz % 128 == 0;
     return balanced_chunk(tiles, c->nz, places, 0.5, !lines ? 2 : (c->f32 ? 5 : 6), cost);
   }
-  return balanced_chunk(tiles, c->nz, places, 4.0, !c->cfg.use_hpml ? c->nz : (c->f32 ? 10 : 5), cost);
+  const int kc = balanced_chunk(tiles, c->nz, places, 4.0, !c->cfg.use_hpml ? c->nz : (c->f32 ? 10 : 5), cost);
+  if (cost) *cost *= std::pow((double)places * tx * ty, large_run(c) ? 1.0 : 0.5);
+  return kc;
 }
 
 // Tile shape, z chunk (kc <= 0: automatic) and the z pass's chunking.
