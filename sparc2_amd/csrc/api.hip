@@ -1677,19 +1677,27 @@ static Shape batch_shape(const std::vector<sparc_ctx*>& runs, const sparc_ctx* c
   return best;
 }
 
-// Planes per z chunk of a run of `tiles` tiles in a batch: its own where it was
-// set, else a rule of the batch's: the runs' items share the persistent blocks,
-// so a run's own rounds do not matter here: 4-plane chunks (MHD xy kernel), or
-// about 512 blocks of at least 2 planes (quiet).
-static int batch_chunk(const sparc_ctx* c, long tiles) {
+// Planes per z chunk of a run in tiles of shape t in a batch: its own where it
+// was set, else a rule of the batch's.  The runs' items share the persistent
+// blocks, so a run's own rounds do not matter here: 4-plane chunks (MHD xy
+// kernel), or about 512 blocks of at least 2 planes (quiet).  Quiet runs with x
+// and y CPML take the chunk they take alone, whose cap evens out the tiles at the
+// sides (six runs with 3-D backgrounds, a stage: FP64 459 us at 512 blocks a run,
+// 345 so; a batch with 256x256x160 1127, 731), FP32 ones no deeper a chunk (six
+// runs 271 at either, 306 at the run's own; with 256x256x160 665, 430).
+static int batch_chunk(const sparc_ctx* c, Shape t) {
   if (!c->kc_auto) return c->kc;
+  const long tiles = (long)((c->nx + t.tx * c->vw - 1) / (t.tx * c->vw)) * ((c->ny + t.ty - 1) / t.ty);
   const long want = c->zp ? 16384 : 512;
-  return (int)std::min<long>(c->nz, std::max<long>(c->zp ? 4 : 2, (c->nz * tiles + want - 1) / want));
+  const int kc = (int)std::min<long>(c->nz, std::max<long>(c->zp ? 4 : 2, (c->nz * tiles + want - 1) / want));
+  if (c->mhd || !c->cfg.use_hpml) return kc;
+  const int alone = auto_chunk(c, t.tx, t.ty, nullptr);
+  return c->f32 ? std::min(kc, alone) : alone;
 }
 
 int sparc_hip_batch_chunk(sparc_ctx* c, int* planes) {
   if (!c || !planes) return fail(SPARC_E_INVALID, "null argument");
-  *planes = batch_chunk(c, (long)c->ntx * c->nty);
+  *planes = batch_chunk(c, {c->tx, c->ty});
   return SPARC_OK;
 }
 
@@ -1756,7 +1764,7 @@ int sparc_hip_batch_create(sparc_ctx* const* runs, int nrun, int use_graph, spar
     g.kc.assign(g.members.size(), 0);
     for (size_t q = 0; q < g.members.size(); ++q) {
       sparc_ctx* c = b->runs[g.members[q]];
-      g.kc[q] = batch_chunk(c, g.ntile[q]);
+      g.kc[q] = batch_chunk(c, {g.tx, g.ty});
       const int items = g.ntile[q] * ((c->nz + g.kc[q] - 1) / g.kc[q]);
       if ((rc = grow_partial(c, items))) return bail(rc);
       b->nblk[g.members[q]] = items;

@@ -46,3 +46,15 @@ def test_tuner_times_deeper_and_deeper_chunks(name, monkeypatch):
     for blocks in timed.values():
         assert len(blocks) == len(batch.KC_MULT)
         assert all(a > b for a, b in zip(blocks, blocks[1:]))
+
+
+@pytest.mark.parametrize("precision,cap", [("fp64", 5), ("fp32", 10)])
+def test_runs_with_open_sides_keep_shallow_chunks_in_a_batch(precision, cap):
+    """512 blocks of this run alone would be 21 (FP64) or 13 planes deep."""
+    from sparc2_amd.solver import Solver
+    cfg = quiet_cfg(nx=150, ny=150, nz=112, periodic=False, use_hpml=True, npml=(6,) * 6, precision=precision)
+    s = Solver(cfg, background(cfg), tile=(32, 8, 0))
+    planes = s.batch_chunk()
+    s.close()
+    print(precision, planes, flush=True)
+    assert 2 <= planes <= cap
