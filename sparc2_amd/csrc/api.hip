@@ -563,20 +563,19 @@ static int balanced_chunk(long tiles, int nz, long places, double c0, int kmax, 
 //    shorter) even that out (192x192x128 FP64 350
 //    us at 36 planes, 227 at 9, 218 at 5; 107x75x117 32x16 81 at 10, 75 at 5);
 //  MHD xy kernel: no window, half a plane to start; at most 6 planes (5 in
-//    FP32), so the halo rows are still in L2 when the neighbouring tiles read
-//    them (256^3 FP64 1484 us at 4 planes, 1473 at 6, 1515 at 12; 64x128x160
-//    FP32, where 5 planes make one round of 512 blocks, 101 us at 4 and 78 at
-//    5), and at most 2 where the tiles' rows share lines with their neighbours
-//    too (191x175x130 FP64 32x8 492 us at 2 planes, 513 at 5; FP32 276 / 299).
+//    FP32).  On large grids the depth hardly matters (256^3 FP64 1433 us at 2
+//    planes, 1432 at 4, 1431 at 6 and 12; 192x192x160 FP64 548, 546, 545, 549,
+//    FP32 302, 300, 301, 303), though the halo rows read twice grow with it
+//    (256^3: 7.3 GB a stage at 4 planes, 7.9 at 6); on small ones rounds decide
+//    (64x128x160 FP32, where 5 planes make one round of 512 blocks, 101 us at 4
+//    and 78 at 5).  At most 2 where the tiles' rows share lines with their
+//    neighbours (191x175x130 FP64 32x8 492 us at 2 planes, 513 at 5; FP32 276 / 299).
 static int auto_chunk(const sparc_ctx* c, int tx, int ty, double* cost) {
   const long tiles = (long)((c->nx + tx * c->vw - 1) / (tx * c->vw)) * ((c->ny + ty - 1) / ty);
   const bool dma = c->dma && tx == 16 && ty == 16;
   const int places = c->f32 ? stage_resident<float>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma)
                             : stage_resident<double>(c->mhd, c->bg3d, c->zp, c->vw, tx, ty, c->ncu, dma);
-  if (c->zp) {
-    const bool lines = (size_t)c->nx * c->esz % 128 == 0;
-    return balanced_chunk(tiles, c->nz, places, 0.5, !lines ? 2 : (c->f32 ? 5 : 6), cost);
-  }
+  if (c->zp) return balanced_chunk(tiles, c->nz, places, 0.5, !whole_lines(c) ? 2 : (c->f32 ? 5 : 6), cost);
   const int kc = balanced_chunk(tiles, c->nz, places, 4.0, !c->cfg.use_hpml ? c->nz : (c->f32 ? 10 : 5), cost);
   if (cost) *cost *= std::pow((double)places * tx * ty, large_run(c) ? 1.0 : 0.5);
   return kc;

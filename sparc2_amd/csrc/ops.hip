@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void k_filter(const T* __restrict__ in, T* __r
 // separate passes, in the same order, so both give the same bits.
 // Bound by the vector instructions in FP32 and on the compensation terms, by
 // memory in FP64.  Five 384x384x160 fields: FP64 729 -> 450 us (1.89 GB), FP32
-// with its compensation 800 -> 575 (1.42 GB); eight of 63x79x101, 7 points,
+// with its compensation 800 -> 560 (1.42 GB); eight of 63x79x101, 7 points,
 // FP64: 61 -> 24.
 constexpr int FXY_PD = 4;
 
