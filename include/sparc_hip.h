@@ -227,7 +227,8 @@ int sparc_hip_get_slab(sparc_ctx* ctx, int field, int k0, int k1, double* out);
 
 /* Batched form: advance many independent runs (contexts on one device, one
  * precision) together.  Each RK stage is one persistent launch per kernel
- * variant and tile shape over the work items of all runs; with use_graph the
+ * variant and tile shape over the work items of all runs (runs of a variant
+ * whose tile is automatic share a shape where one fits them all); with use_graph the
  * launch sequence of one step is captured once in a HIP graph and replayed.
  * No counterpart in the reference (one run per MPI job there); it serves
  * callers that run many forward simulations at once.
